@@ -35,6 +35,7 @@ SOURCES = [
     "envmap_kernels.hip",
     "encode_kernels.hip",
     "relight_kernels.hip",
+    "relight_f32_kernels.hip",
     "relight_fp8_kernels.hip",
     "denoise_kernels.hip",
     "gbuffer_kernels.hip",

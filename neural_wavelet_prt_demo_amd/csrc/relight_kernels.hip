@@ -115,102 +115,7 @@ __global__ __launch_bounds__(kRelightBlock, MINW) void relight_batch_kernel(
 
 __global__ void reset_counter_kernel(unsigned int *counter) { *counter = 0u; }
 
-// Plain FP32 form: one lane per pixel walks the K wavelets with the four
-// layers on the vector ALU, weights broadcast from LDS and the selected
-// wavelet features read with uniform (scalar) loads.
-constexpr int kPlainBlock = 256;
-constexpr int kW1 = 64 * 32, kW2 = 64 * 64, kW3 = 64 * 64, kW4 = 3 * 64;
-
-constexpr int kWaux = 64 * 16;
-
-template <bool DUMP, bool AUX>
-__global__ __launch_bounds__(kPlainBlock) void relight_plain_kernel(RelightArgs a) {
-  __shared__ float w[kW1 + kW2 + kW3 + kW4 + (AUX ? kWaux : 0)];
-  for (int i = threadIdx.x; i < kW1 + kW2 + kW3 + kW4; i += kPlainBlock) w[i] = a.w_f32[i];
-  if (AUX)
-    for (int i = threadIdx.x; i < kWaux; i += kPlainBlock) w[kW1 + kW2 + kW3 + kW4 + i] = a.waux_f32[i];
-  __syncthreads();
-  const int p = blockIdx.x * kPlainBlock + threadIdx.x;
-  if (p >= a.n_pixels) return;
-  const bool hit = a.env_flag == nullptr || a.env_flag[p] != 0;
-  float sum[3] = {0.f, 0.f, 0.f}, comp[3] = {0.f, 0.f, 0.f}, pend[3] = {0.f, 0.f, 0.f};
-  if (hit) {
-    float h[32];
-    const float4 *fp = (const float4 *)((const float *)a.features + (size_t)p * 32);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float4 v = fp[q];
-      h[4 * q] = v.x; h[4 * q + 1] = v.y; h[4 * q + 2] = v.z; h[4 * q + 3] = v.w;
-    }
-    // Aux inputs enter the second layer as a per-pixel constant term.
-    float b2[64];
-#pragma unroll
-    for (int o = 0; o < 64; ++o) b2[o] = 0.f;
-    if (AUX) {
-      const float *ax = (const float *)a.aux + (size_t)p * 16;
-      const float *Wa = w + kW1 + kW2 + kW3 + kW4;
-#pragma unroll
-      for (int o = 0; o < 64; ++o) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc = fmaf(Wa[o * 16 + i], ax[i], acc);
-        b2[o] = acc;
-      }
-    }
-    for (int k = 0; k < a.k; ++k) {
-      // The weight reads are loop-invariant; an opaque zero offset keeps the
-      // compiler from hoisting all ~10K of them out of the K loop.
-      int wo = 0;
-      asm volatile("" : "+s"(wo));
-      const float *W1 = w + wo, *W2 = W1 + kW1, *W3 = W2 + kW2, *W4 = W3 + kW3;
-      const float *ws = a.wsel + (size_t)k * 32;
-      float y1[64];
-#pragma unroll
-      for (int o = 0; o < 64; ++o) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) acc = fmaf(W1[o * 32 + i], h[i] * ws[i], acc);
-        y1[o] = fmaxf(acc, 0.f);
-      }
-      float y2[64];
-#pragma unroll
-      for (int o = 0; o < 64; ++o) {
-        float acc = b2[o];
-#pragma unroll
-        for (int i = 0; i < 64; ++i) acc = fmaf(W2[o * 64 + i], y1[i], acc);
-        y2[o] = fmaxf(acc, 0.f);
-      }
-#pragma unroll
-      for (int o = 0; o < 64; ++o) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < 64; ++i) acc = fmaf(W3[o * 64 + i], y2[i], acc);
-        y1[o] = fmaxf(acc, 0.f);  // reuse y1 as layer-3 output
-      }
-#pragma unroll
-      for (int ch = 0; ch < 3; ++ch) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < 64; ++i) acc = fmaf(W4[ch * 64 + i], y1[i], acc);
-        const float t = a.softplus ? dev::softplus(acc) : acc;
-        // Pairs of wavelets: the clamped terms of k and k + 1 are added and
-        // the pair sum enters the compensated running sum (the fused kernel's
-        // order).
-        const float term = dev::relu_f32(a.light[3 * k + ch] * t);
-        if (k & 1) dev::neumaier_add(sum[ch], comp[ch], pend[ch] + term);
-        else pend[ch] = term;
-        if (DUMP) {
-          const int q = p - a.dump_begin;
-          if (q >= 0 && q < a.dump_count) a.dump[((size_t)q * a.k + k) * 3 + ch] = t;
-        }
-      }
-    }
-    if (a.k & 1)
-      for (int ch = 0; ch < 3; ++ch) dev::neumaier_add(sum[ch], comp[ch], pend[ch]);
-  }
-  write_outputs(a, p, hit ? sum[0] + comp[0] : 0.f, hit ? sum[1] + comp[1] : 0.f,
-                hit ? sum[2] + comp[2] : 0.f);
-}
+constexpr int kW1 = 64 * 32, kW2 = 64 * 64, kW3 = 64 * 64;
 
 // Activation calibration for the FP8 form: the BF16 network over a pixel
 // subsample (a.features, a.n_pixels) and the wavelets [k0, k0 + k_chunk) of
@@ -497,23 +402,6 @@ void launch_relight_mfma(const RelightArgs &a, Elem elem, int variant, hipStream
     fail(NWPRT_ERR_INVALID_ARGUMENT, "relight: MFMA element must be BF16 or FP16");
   }
   hip_check(hipGetLastError(), "relight_mfma_kernel launch");
-}
-
-void launch_relight_plain(const RelightArgs &a, hipStream_t s) {
-  require(a.n_pixels >= 1 && a.k >= 1 && a.k <= NWPRT_MAX_K, NWPRT_ERR_INVALID_ARGUMENT,
-          "relight: bad pixel count or K");
-  require(a.features && a.wsel && a.light && a.w_f32 && a.direct, NWPRT_ERR_INVALID_ARGUMENT,
-          "relight: missing operand");
-  const dim3 grid((a.n_pixels + kPlainBlock - 1) / kPlainBlock), block(kPlainBlock);
-  if (a.aux) {
-    require(a.waux_f32 != nullptr, NWPRT_ERR_INVALID_ARGUMENT, "relight: missing aux weights");
-    if (a.dump) hipLaunchKernelGGL((relight_plain_kernel<true, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((relight_plain_kernel<false, true>), grid, block, 0, s, a);
-  } else {
-    if (a.dump) hipLaunchKernelGGL((relight_plain_kernel<true, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((relight_plain_kernel<false, false>), grid, block, 0, s, a);
-  }
-  hip_check(hipGetLastError(), "relight_plain_kernel launch");
 }
 
 bool relight_batch_variant_ok(int v) {
