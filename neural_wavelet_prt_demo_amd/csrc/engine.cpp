@@ -331,14 +331,14 @@ std::tuple<int, int, int> tune_key(nwprt_precision prec, int k, int n_pixels) {
 }
 
 // Kernel variant for a relight: the forced one (BF16 / FP16 only), else the
-// autotuner's choice for this shape bucket, else 0.
+// autotuner's choice for this shape bucket, else the form's default.
 int pick_variant(nwprt_ctx ctx, nwprt_precision prec, int k, int n_pixels) {
   if (ctx->forced_variant >= 0 &&
       (prec != NWPRT_PREC_FP8 || ctx->forced_variant < relight_fp8_variant_count()))
     return ctx->forced_variant;
   auto it = ctx->tuned.find(tune_key(prec, k, n_pixels));
   if (it != ctx->tuned.end()) return it->second;
-  return prec == NWPRT_PREC_FP8 ? kDefaultFp8Variant : 0;
+  return prec == NWPRT_PREC_FP8 ? kDefaultFp8Variant : kDefaultMfmaVariant;
 }
 
 int variant_count(nwprt_precision prec) {

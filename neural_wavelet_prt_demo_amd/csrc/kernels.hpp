@@ -138,6 +138,7 @@ struct RelightArgs {
   nwprt_hashgrid_levels lv;
 };
 // Tile-shape variants of the fused kernel (see relight_kernels.hip).
+constexpr int kDefaultMfmaVariant = 5;  // pipe.w4reg.occ2
 int relight_mfma_variant_count();
 const char *relight_mfma_variant_name(int variant);
 void launch_relight_mfma(const RelightArgs &a, Elem elem, int variant, hipStream_t s);

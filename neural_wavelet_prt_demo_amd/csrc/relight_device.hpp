@@ -69,6 +69,15 @@ struct LightTerm {
     const float sp = __builtin_amdgcn_logf(1.0f + __builtin_amdgcn_exp2f(y));
     return o > 15.0f ? y : sp;
   }
+  // The pair of wavelets (k, k + 1): term(first) + term(second) from the lights
+  // and values (`value`), the second product fused into the addition.
+  __device__ static __forceinline__ float value(float o) { return SOFTPLUS ? factor(o) : o; }
+  __device__ static __forceinline__ float first(float light, float v) {
+    return SOFTPLUS ? light * v : relu_f32(light * v);
+  }
+  __device__ static __forceinline__ float second(float x, float light, float v) {
+    return SOFTPLUS ? fmaf(light, v, x) : x + relu_f32(light * v);
+  }
   // Per pair: the term divided by kSumScale.
   __device__ static __forceinline__ float term(float light, float o) {
     if constexpr (SOFTPLUS) {
@@ -120,6 +129,36 @@ __device__ __forceinline__ void encode_batch(const RelightArgs &a, int l0, const
     pk[l < 8 ? 2 * l : 2 * (15 - l) + 1] = std::is_same<E, _Float16>::value
                                                 ? pack_f16_rounded(v[i][0], v[i][1])
                                                 : pack_bf16(v[i][0], v[i][1]);
+  }
+}
+
+// Levels 4 part .. 4 part + 3 of pixel my_px into words of its 64 B row of
+// `lds`, as fused_encode_lds stores them: the four waves of a workgroup that
+// share 64 pixels encode a quarter of the levels each.  The caller's barrier
+// orders the stores before the loads.
+template <typename E>
+__device__ __forceinline__ void fused_encode_part(const RelightArgs &a, bool active, int my_px,
+                                                  int lane, int part, uint32_t *lds) {
+  uint32_t pk[4] = {0u, 0u, 0u, 0u};
+  const int l0 = 4 * part;
+  if (active) {
+    const f32x4 x4 = *(gptr<f32x4>)(a.position + 4 * (size_t)my_px);
+    const float x[3] = {x4[0], x4[1], x4[2]};
+    float v[4][2];
+    if (a.hash_f16) {
+      gather_levels<4, true>(a.lv, a.hash, l0, x, v);
+    } else {
+      gather_levels<4, false>(a.lv, a.hash, l0, x, v);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      pk[i] = std::is_same<E, _Float16>::value ? pack_f16_rounded(v[i][0], v[i][1])
+                                               : pack_bf16(v[i][0], v[i][1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int l = l0 + i;
+    lds[lane * 16 + (l < 8 ? 2 * l : 2 * (15 - l) + 1)] = pk[i];
   }
 }
 

@@ -52,20 +52,46 @@ constexpr MfmaVariant kMfmaVariants[] = {
 };
 constexpr int kNumMfmaVariants = sizeof(kMfmaVariants) / sizeof(kMfmaVariants[0]);
 
-// Grid: ceil(P / 256) workgroups of 4 waves; wave w of the workgroup with
+// Workgroups that take 256 pixels (64 a wave) before the ones that take 64
+// together (relight_group).  The chip holds 512 workgroups of these kernels
+// (256 CUs, two waves a SIMD).  Whole rounds of 512 go 64 pixels a wave; the
+// rest of the frame, at most one round, is split finer unless it fills more
+// than three quarters of a round, where the finer form's four quarter rounds
+// would take longer than the one it replaces.  Measured, whole requests: 128 x
+// 128, K = 64, BF16 (64 workgroups before, 256 now) 142 -> 73 us; 1283 x 717,
+// K = 128, FP16 (7.02 rounds) 1875 -> 1705 us, half of it the pipelined step
+// becoming the untuned default (1920 x 1080, K = 300: 9423 -> 9145 us).
+constexpr int kRoundWgs = 512;
+int full_workgroups(int n_pixels) {
+  const int wgs = (n_pixels + kRelightBlock - 1) / kRelightBlock;
+  const int rest = wgs % kRoundWgs;
+  return 4 * rest > 3 * kRoundWgs ? wgs : wgs - rest;
+}
+
+// Grid: `full` workgroups of 4 waves x 64 pixels -- wave w of the one with
 // tile t = xcd_tile(b) owns pixels [64 (4 t + w), +64), so each XCD relights
-// (and with the fused encode, gathers hash entries for) one contiguous band.
-template <typename E, bool SOFTPLUS, bool DUMP, bool AUX, int GP, bool W4LDS, int MINW>
-__global__ __launch_bounds__(kRelightBlock, MINW) void relight_mfma_kernel(RelightArgs a) {
+// (and with the fused encode, gathers hash entries for) one contiguous band --
+// then, in the instances with SPLIT, workgroups whose waves share 64 pixels.
+template <typename E, bool SOFTPLUS, bool DUMP, bool AUX, int GP, bool W4LDS, int MINW, bool SPLIT>
+__global__ __launch_bounds__(kRelightBlock, MINW) void relight_mfma_kernel(RelightArgs a,
+                                                                           int full) {
   __shared__ u32x4 w4s[W4LDS ? 4 * 2 * 64 : 1];
-  __shared__ uint32_t feat_lds[AUX ? 1 : 4 * 64 * 16];  // fused encode: [wave][pixel][16]
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // Fused encode: [wave][pixel][16]; a sharing workgroup's features and terms.
+  __shared__ uint32_t feat_lds[AUX ? (SPLIT ? kGroupLdsWords : 1) : 4 * 64 * 16];
+  static_assert(kGroupLdsWords <= 4 * 64 * 16, "a sharing workgroup's LDS fits the waves' rows");
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (SPLIT && (int)blockIdx.x >= full) {
+    const int tail = (int)gridDim.x - full;
+    const int base = full * kRelightBlock + dev::xcd_tile((int)blockIdx.x - full, tail) * 64;
+    relight_group<E, SOFTPLUS, AUX, !AUX>(a, base, wave, lane, feat_lds);
+    return;
+  }
   if (W4LDS) {
     const u32x4 *wt = (const u32x4 *)a.w_tiles;
     for (int i = threadIdx.x; i < 4 * 2 * 64; i += kRelightBlock) w4s[i] = wt[2 * 8 * 64 + i];
     __syncthreads();
   }
-  const int base = (dev::xcd_tile(blockIdx.x, gridDim.x) * 4 + wave) * 64;
+  const int base = (dev::xcd_tile(blockIdx.x, full) * 4 + wave) * 64;
   if (base >= a.n_pixels) return;
   relight_wave<E, SOFTPLUS, DUMP, AUX, GP, W4LDS, !AUX>(a, base, lane, w4s,
                                                        feat_lds + (AUX ? 0 : wave * 64 * 16));
@@ -271,37 +297,40 @@ __global__ __launch_bounds__(256) void tonemap_kernel(const float *__restrict__ 
   dst[p] = dev::tonemap_rgba8(v.x, v.y, v.z);
 }
 
+template <typename E, bool SP, bool DUMP, bool AUX, int GP, bool W4LDS, int MINW, bool SPLIT>
+void launch_shape(const RelightArgs &a, hipStream_t s) {
+  const int wgs = (a.n_pixels + kRelightBlock - 1) / kRelightBlock;
+  const int full = SPLIT ? full_workgroups(a.n_pixels) : wgs;
+  const int rest = full < wgs ? a.n_pixels - full * kRelightBlock : 0;
+  hipLaunchKernelGGL((relight_mfma_kernel<E, SP, DUMP, AUX, GP, W4LDS, MINW, SPLIT>),
+                     dim3(full + (rest + 63) / 64), dim3(kRelightBlock), 0, s, a, full);
+}
+
 template <typename E, bool SP, int V>
-void launch_v(const RelightArgs &a, dim3 grid, dim3 block, hipStream_t s) {
+void launch_v(const RelightArgs &a, hipStream_t s) {
   constexpr MfmaVariant v = kMfmaVariants[V];
   if (a.aux) {
-    // Aux scenes are built for variant 0's tile shape (tap included).
-    if (a.dump)
-      hipLaunchKernelGGL((relight_mfma_kernel<E, SP, true, true, 2, false, 2>), grid, block, 0, s, a);
-    else
-      hipLaunchKernelGGL((relight_mfma_kernel<E, SP, false, true, 2, false, 2>), grid, block, 0, s,
-                         a);
+    // Aux scenes are built for one tile shape (and variant 0's for the tap).
+    if (a.dump) launch_shape<E, SP, true, true, 2, false, 2, false>(a, s);
+    else launch_shape<E, SP, false, true, 2, false, 2, true>(a, s);
   } else if (a.dump && V == 0) {
-    hipLaunchKernelGGL((relight_mfma_kernel<E, SP, true, false, v.gp, v.w4_lds, v.min_waves>),
-                       grid, block, 0, s, a);
+    launch_shape<E, SP, true, false, v.gp, v.w4_lds, v.min_waves, false>(a, s);
   } else {
-    hipLaunchKernelGGL((relight_mfma_kernel<E, SP, false, false, v.gp, v.w4_lds, v.min_waves>),
-                       grid, block, 0, s, a);
+    launch_shape<E, SP, false, false, v.gp, v.w4_lds, v.min_waves, V == kDefaultMfmaVariant>(a, s);
   }
 }
 
 template <typename E, bool SP>
 void launch_sp(const RelightArgs &a, int variant, hipStream_t s) {
-  const dim3 grid((a.n_pixels + kRelightBlock - 1) / kRelightBlock), block(kRelightBlock);
   if (a.dump) variant = 0;  // the transport tap is built for the default variant only
   switch (variant) {
-    case 0: launch_v<E, SP, 0>(a, grid, block, s); break;
-    case 1: launch_v<E, SP, 1>(a, grid, block, s); break;
-    case 2: launch_v<E, SP, 2>(a, grid, block, s); break;
-    case 3: launch_v<E, SP, 3>(a, grid, block, s); break;
-    case 4: launch_v<E, SP, 4>(a, grid, block, s); break;
-    case 5: launch_v<E, SP, 5>(a, grid, block, s); break;
-    case 6: launch_v<E, SP, 6>(a, grid, block, s); break;
+    case 0: launch_v<E, SP, 0>(a, s); break;
+    case 1: launch_v<E, SP, 1>(a, s); break;
+    case 2: launch_v<E, SP, 2>(a, s); break;
+    case 3: launch_v<E, SP, 3>(a, s); break;
+    case 4: launch_v<E, SP, 4>(a, s); break;
+    case 5: launch_v<E, SP, 5>(a, s); break;
+    case 6: launch_v<E, SP, 6>(a, s); break;
     default: fail(NWPRT_ERR_INVALID_ARGUMENT, "relight: unknown kernel variant");
   }
 }

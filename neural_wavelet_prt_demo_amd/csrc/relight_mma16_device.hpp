@@ -313,8 +313,10 @@ __device__ __forceinline__ void relight_wave(const RelightArgs &a, int base, int
       }
 #pragma unroll
       for (int ch = 0; ch < 3; ++ch) {
-        float x = LT::term(LT::light(dev::load_invariant(a.light + 3 * k + ch)), o0[ch]);
-        if (two) x += LT::term(LT::light(dev::load_invariant(a.light + 3 * (k + 1) + ch)), o1[ch]);
+        float x = LT::first(LT::light(dev::load_invariant(a.light + 3 * k + ch)), LT::value(o0[ch]));
+        if (two)
+          x = LT::second(x, LT::light(dev::load_invariant(a.light + 3 * (k + 1) + ch)),
+                         LT::value(o1[ch]));
         dev::kahan_add(sum[ch], comp[ch], x);
         if (DUMP) {
           const int q = my_px - a.dump_begin;
@@ -332,6 +334,112 @@ __device__ __forceinline__ void relight_wave(const RelightArgs &a, int base, int
                 bb = hit ? (sum[2] - comp[2]) * f : 0.f;
     write_outputs(a, my_px, r, gg, bb);
   }
+}
+
+// The workgroup form: four waves share the 64 pixels [base, base + 64), wave w
+// taking wavelets 4 r + w of round r (the pipelined step; with aux inputs the
+// two-group one, as relight_wave takes them).  The round's
+// outputs meet in LDS (two buffers, one barrier a round); wave c < 3 adds
+// channel c's terms in wavelet order, so every pixel's sum is relight_wave's,
+// bit for bit.  The waves also split the fused encode, four levels each.  A
+// group of 64 pixels takes about a quarter of relight_wave's time on four
+// times the waves.  `lds`: 4 KB features, then 6 KB of terms.
+constexpr int kGroupWaves = 4;
+constexpr int kGroupLdsWords = 64 * 16 + 2 * kGroupWaves * 3 * 64;
+template <typename E, bool SOFTPLUS, bool AUX, bool FUSE>
+__device__ __forceinline__ void relight_group(const RelightArgs &a, int base, int wave, int lane,
+                                              uint32_t *lds) {
+  const int g = lane >> 4, n = lane & 15;
+  const int P = a.n_pixels;
+  const int my_px = base + lane;
+  const bool mine = my_px < P;
+  const bool hit =
+      mine && (a.env_flag == nullptr || *((dev::gptr<uint8_t>)a.env_flag + my_px) != 0);
+  float *terms = (float *)(lds + 64 * 16);
+  float rgb[3] = {0.f, 0.f, 0.f};
+  if (__ballot(hit) != 0) {  // uniform over the workgroup: its waves see the same pixels
+    u32x4 hb[4];
+    if (FUSE && a.fused_encode) {
+      dev::fused_encode_part<E>(a, hit, my_px, lane, wave, lds);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) hb[j] = *(const u32x4 *)(lds + (16 * j + n) * 16 + 4 * g);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int p = base + 16 * j + n;
+        hb[j] = p < P ? dev::load_features8(a, P, p, 8 * g) : u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+    u32x2 auxb[4], waux[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int p = base + 16 * j + n;
+      auxb[j] = AUX && p < P ? *(const u32x2 *)((const uint16_t *)a.aux + (size_t)p * 16 + 4 * g)
+                             : u32x2{0u, 0u};
+      waux[j] = AUX ? ((const u32x2 *)a.waux_tiles)[j * 64 + lane] : u32x2{0u, 0u};
+    }
+    const dev::gptr<u32x4> wt = (dev::gptr<u32x4>)a.w_tiles;
+    u32x4 w2[4][2], w3[4][2], w4[4][2];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        w2[b][kb] = wt[(0 * 8 + b * 2 + kb) * 64 + lane];
+        w3[b][kb] = wt[(1 * 8 + b * 2 + kb) * 64 + lane];
+        w4[b][kb] = wt[(2 * 8 + b * 2 + kb) * 64 + lane];
+      }
+    const dev::gptr<u32x4> mk = (dev::gptr<u32x4>)a.mk;
+    u32x4 ta[4];
+    if (wave < a.k) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) ta[b] = mk[((size_t)wave * 4 + b) * 64 + lane];
+    }
+    using LT = dev::LightTerm<SOFTPLUS>;
+    float sum = 0.f, comp = 0.f;  // channel `wave`
+    for (int k0 = 0; k0 < a.k; k0 += kGroupWaves) {
+      const int k = k0 + wave;
+      float *buf = terms + (k0 / kGroupWaves & 1) * kGroupWaves * 3 * 64;
+      if (k < a.k) {
+        u32x4 t[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) t[b] = ta[b];
+        if (k + kGroupWaves < a.k) {
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            ta[b] = mk[((size_t)(k + kGroupWaves) * 4 + b) * 64 + lane];
+        }
+        f32x4 o;
+        if constexpr (AUX)
+          o = wavelet_step<E, true, 2, false>(t, hb, auxb, waux, w2, w3, w4, nullptr, lane);
+        else
+          o = wavelet_step_pipelined<E, false, false>(t, hb, auxb, waux, w2, w3, w4, nullptr, lane);
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) buf[(wave * 3 + ch) * 64 + lane] = LT::value(o[ch]);
+      }
+      __syncthreads();
+      if (wave < 3) {
+#pragma unroll
+        for (int q = 0; q < kGroupWaves; q += 2) {
+          const int kq = k0 + q;
+          if (kq >= a.k) break;
+          float x = LT::first(LT::light(dev::load_invariant(a.light + 3 * kq + wave)),
+                              buf[(q * 3 + wave) * 64 + lane]);
+          if (kq + 1 < a.k)
+            x = LT::second(x, LT::light(dev::load_invariant(a.light + 3 * (kq + 1) + wave)),
+                           buf[((q + 1) * 3 + wave) * 64 + lane]);
+          dev::kahan_add(sum, comp, x);
+        }
+      }
+    }
+    // The channels meet in the first buffer once its last round is read.
+    __syncthreads();
+    if (wave < 3) terms[wave * 64 + lane] = (sum - comp) * LT::kSumScale;
+    __syncthreads();
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) rgb[ch] = hit ? terms[ch * 64 + lane] : 0.f;
+  }
+  if (mine && wave == 0) write_outputs(a, my_px, rgb[0], rgb[1], rgb[2]);
 }
 
 }  // namespace mma16
