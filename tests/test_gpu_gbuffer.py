@@ -137,6 +137,27 @@ def test_cast_small_and_degenerate_meshes(nw, orc, ctx, nt):
     _compare(got, want)
 
 
+@pytest.mark.parametrize("leaf", [1, 3, 8])
+def test_cast_skewed_tree(nw, orc, ctx, leaf):
+    # Groups of `leaf` parallel triangles whose size grows by 1.6 a group, all
+    # around one axis: the surface-area split peels one group off a level, so a
+    # ray near the axis leaves an entry on its stack at most levels of the
+    # tree and takes leaves of few triangles up to the largest.
+    base = np.array([[-1, -1, 0], [1, -1, 0], [0, 1.5, 0]], np.float64)
+    v = np.concatenate([base * 0.05 * 1.6 ** i + [0, 0, -3 - 0.01 * 1.6 ** i - 0.002 * j]
+                        for i in range(22) for j in range(leaf)])
+    nt = 22 * leaf
+    s = {"vertices": v.astype(np.float32),
+         "indices": np.arange(3 * nt, dtype=np.int32).reshape(-1, 3),
+         "materials": np.array([[0.2, 0.3, 0.4, 0.0, 0.0, 0.0, 0.6, 0]], np.float32),
+         "camera": [0.0, 0.0, 2.0, 0.0, 0.0, -1.0, 0.0, 1.0, 0.0],
+         "bounds": np.array([-2000, -2000, -500, 2000, 3000, 10], np.float32)}
+    got, info = _cast(nw, ctx, s, 41, 33)
+    want = _oracle(orc, s, 41, 33)
+    _compare(got, want)
+    assert 4 <= info["bvh_depth"] <= 24
+
+
 def test_cast_null_fields_are_skipped(nw, ctx):
     s = mesh_scene(3)
     mesh = ctx.mesh_create(s["vertices"], s["indices"], s["materials"], normals=s["normals"],
