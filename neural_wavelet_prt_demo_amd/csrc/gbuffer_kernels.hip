@@ -821,6 +821,7 @@ __host__ __device__ inline size_t env_face_doubles(int n) {
   return (size_t)n * (n + 1) + (size_t)n * n + (n + 1) + n;
 }
 constexpr int kTabHead = 19;
+__host__ __device__ inline size_t table_doubles(int n) { return kTabHead + 6 * env_face_doubles(n); }
 
 // First index i in [0, count) with cdf[i] > r (count when none), as the
 // linear searches of cubeMap.cu:115-164 find it.
@@ -929,10 +930,15 @@ __device__ float3 direct_light(const CastArgs &a, const Surface &s, float3 p, fl
 // Pass 1: one workgroup per (face, row), one lane per texel; the row's
 // prefix sum runs in order on lane 0.  The row integral and the row's raw
 // luminance sum are parked in the face's marginal arrays for pass 2.
+// The grid's second dimension (here and in pass 2; the first in pass 3) is the
+// map: the basis maps of a transfer computation take three launches together,
+// not three each (25 maps: 0.42 -> 0.03 ms).
 __global__ __launch_bounds__(128) void env_rows_kernel(const float *__restrict__ faces, int n,
                                                       double *__restrict__ tab) {
 #pragma clang fp contract(off)
   const int f = blockIdx.x / n, r = blockIdx.x % n, c = threadIdx.x;
+  faces += (size_t)blockIdx.y * 6 * n * n * 3;
+  tab += (size_t)blockIdx.y * table_doubles(n);
   double *base = tab + kTabHead + (size_t)f * env_face_doubles(n);
   double *cr = base + (size_t)r * (n + 1);
   double *pr = base + (size_t)n * (n + 1) + (size_t)r * n;
@@ -984,6 +990,7 @@ __global__ __launch_bounds__(128) void env_rows_kernel(const float *__restrict__
 __global__ __launch_bounds__(128) void env_marginals_kernel(int n, double *__restrict__ tab) {
 #pragma clang fp contract(off)
   const int f = blockIdx.x, r = threadIdx.x;
+  tab += (size_t)blockIdx.y * table_doubles(n);
   double *base = tab + kTabHead + (size_t)f * env_face_doubles(n);
   double *cdf_m = base + (size_t)n * (n + 1) + (size_t)n * n, *pdf_m = cdf_m + (n + 1);
   __shared__ double row_int[128], row_lum[128];
@@ -1021,9 +1028,10 @@ __global__ __launch_bounds__(128) void env_marginals_kernel(int n, double *__res
 
 // Face distribution (EnvironmentMap.cpp:180-189, make_table_dist_1d,
 // table_dist.cpp:4-27); an all-black map gets the uniform distribution.
-__global__ void env_face_table_kernel(double *__restrict__ tab) {
+__global__ void env_face_table_kernel(int n, double *__restrict__ tab) {
 #pragma clang fp contract(off)
   if (threadIdx.x != 0) return;
+  tab += (size_t)blockIdx.x * table_doubles(n);
   double total = 0.0, f[6];
   for (int i = 0; i < 6; ++i) total += tab[13 + i];
   for (int i = 0; i < 6; ++i) f[i] = total > 0 ? tab[13 + i] / total : 0.0;
@@ -1226,10 +1234,12 @@ __device__ inline void sh_eval(float3 w, float (&y)[kShCoeffs]) {
   }
 }
 
-// R[v][k] = sum_j T[v][k][j] (x) L[j].  One wavefront per vertex walks its
-// nc rows; a row's nc x 3 floats are read by the 64 lanes together
+// R[v][k] = sum_j T[v][k][j] (x) L[j].  A workgroup per vertex, a quarter of
+// its nc rows a wave; a row's nc x 3 floats are read by the 64 lanes together
 // (coalesced) and multiplied by L flattened the same way, then reduced
-// across the wave per channel.  Four vertices per 256-thread workgroup.
+// across the wave per channel.  Bound: HBM (18.6 K vertices of degree 8, 1.47 GB:
+// 345 us with a vertex a wave, 2.3 rounds of the chip's waves, 323 us so split;
+// 4.5 TB/s, a large copy's rate is 5.0).
 __device__ inline float wave_sum(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -1248,8 +1258,9 @@ static_assert((kShMaxDegree + 1) * (kShMaxDegree + 1) * 3 <= 64 * kShRowSlots,
 __global__ __launch_bounds__(256) void sh_light_response_kernel(ShArgs a) {
   const int nc = (a.degree + 1) * (a.degree + 1), row = nc * 3;
   const int lane = threadIdx.x & 63;
-  const long long v = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (v >= a.n_vertices) return;  // whole waves leave together; no barriers below
+  const long long v = blockIdx.x;
+  const int per = (nc + 3) / 4;  // rows a wave
+  const int kb = per * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ke = min(kb + per, nc);
   const float *t = a.transfer + (size_t)v * nc * row;
   float *o = a.light_response + (size_t)v * row;
   float l[kShRowSlots];
@@ -1265,12 +1276,12 @@ __global__ __launch_bounds__(256) void sh_light_response_kernel(ShArgs a) {
 #pragma unroll
     for (int s = 0; s < kShRowSlots; ++s) {
       const int f = lane + 64 * s;
-      r[s] = (k < nc && f < row) ? t[(size_t)k * row + f] : 0.0f;
+      r[s] = (k < ke && f < row) ? t[(size_t)k * row + f] : 0.0f;
     }
   };
 #pragma unroll
-  for (int d = 0; d < kShRowsInFlight; ++d) load_row(d, buf[d]);
-  for (int k0 = 0; k0 < nc; k0 += kShRowsInFlight) {
+  for (int d = 0; d < kShRowsInFlight; ++d) load_row(kb + d, buf[d]);
+  for (int k0 = kb; k0 < ke; k0 += kShRowsInFlight) {
 #pragma unroll
     for (int d = 0; d < kShRowsInFlight; ++d) {
       float cur[kShRowSlots];
@@ -1278,7 +1289,7 @@ __global__ __launch_bounds__(256) void sh_light_response_kernel(ShArgs a) {
       for (int s = 0; s < kShRowSlots; ++s) cur[s] = buf[d][s];
       load_row(k0 + kShRowsInFlight + d, buf[d]);
       const int k = k0 + d;
-      if (k >= nc) continue;  // wave-uniform
+      if (k >= ke) continue;  // wave-uniform
       float acc0 = 0.0f, acc1 = 0.0f, acc2 = 0.0f;
 #pragma unroll
       for (int s = 0; s < kShRowSlots; ++s) {
@@ -1710,65 +1721,79 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void tm
   o[2] = color.z - tent.z;
 }
 
-// The projection stages the filtered basis of 64 samples at a time in LDS;
-// lane (map, channel) then walks them in sample order.
-constexpr int kTmProjectSamples = 64;
-
+// The projection of one vertex, T[k][col] = sum over samples of y[j][k] x[j][col],
+// in sample order.  Thread (group g, col) carries KPT rows k = KPT g .. of one
+// (map, channel) column; the basis and the scaled indirect radiance of CHUNK
+// samples at a time are staged in LDS, where a NaN map of a sample is marked
+// by a NaN in all three of its channels.  Bound: HBM reads of the two arrays,
+// with the loads of a chunk issued together (one thread a column, reading its
+// samples one after the other, ran at the latency of those loads: 2116 vertices,
+// 64 samples, degree 4: 831 -> 41 us).
+template <int KPT, int CHUNK>
 __global__ __launch_bounds__(256) void tm_project_kernel(TmArgs a) {
-  __shared__ float ylds[kTmProjectSamples][kTmRow];
+  constexpr int kMaxCols = KPT > 9 ? 3 * kShCoeffs : 75;
+  __shared__ float ylds[CHUNK * kTmRow];
+  __shared__ float xlds[CHUNK * kMaxCols];
   const int t = threadIdx.x;
   const int nc = (a.degree + 1) * (a.degree + 1), cols = 3 * nc;
   const long long vl = blockIdx.x;
   const long long pairs = a.n_verts * a.samples;
   const TmWork w = tm_work(a.work, pairs, tm_slots(a.max_bounce), nc);
   const float *ind = w.ind + (size_t)vl * a.samples * cols;
+  const float *ysrc = w.y + (size_t)vl * a.samples * kTmRow;
   const float fn = (float)a.samples, scale_n = 4.0f * 3.14159265358979f / fn;
-  float acc[kShCoeffs];
+  const int g = t / cols, col = t - g * cols, k0 = g * KPT;
+  const bool live = k0 < nc;
+  float acc[KPT];
 #pragma unroll
-  for (int k = 0; k < kShCoeffs; ++k) acc[k] = 0.0f;
-  const int i = t / 3;
-  for (int s0 = 0; s0 < a.samples; s0 += kTmProjectSamples) {
-    const int m = min(kTmProjectSamples, a.samples - s0);
+  for (int k = 0; k < KPT; ++k) acc[k] = 0.0f;
+  for (int s0 = 0; s0 < a.samples; s0 += CHUNK) {
+    const int m = min(CHUNK, a.samples - s0);
     __syncthreads();
-    const float *ysrc = w.y + ((size_t)vl * a.samples + s0) * kTmRow;
-    for (int e = t; e < m * kTmRow; e += 256) (&ylds[0][0])[e] = ysrc[e];
+    for (int e = t; e < m * kTmRow; e += 256) ylds[e] = ysrc[(size_t)s0 * kTmRow + e];
+    // A map's three channels by one thread.
+    for (int e = t; e < m * nc; e += 256) {
+      const float *x = ind + (size_t)s0 * cols + 3 * (size_t)e;
+      const float r = x[0], gg = x[1], b = x[2];
+      const bool bad = isnan(r) || isnan(gg) || isnan(b);
+      xlds[3 * e] = bad ? NAN : r * scale_n;
+      xlds[3 * e + 1] = bad ? NAN : gg * scale_n;
+      xlds[3 * e + 2] = bad ? NAN : b * scale_n;
+    }
     __syncthreads();
-    if (t < cols) {
+    if (live) {
       for (int j = 0; j < m; ++j) {
-        const float *row = ind + (size_t)(s0 + j) * cols;
-        const float x = row[t] * scale_n;
-        if (isnan(row[3 * i]) || isnan(row[3 * i + 1]) || isnan(row[3 * i + 2])) {
+        const float x = xlds[j * cols + col];
+        if (isnan(x)) {
 #pragma unroll
-          for (int k = 0; k < kShCoeffs; ++k)
-            if (k < nc) acc[k] += acc[k] / fn;
+          for (int k = 0; k < KPT; ++k) acc[k] += acc[k] / fn;
         } else {
 #pragma unroll
-          for (int k = 0; k < kShCoeffs; ++k)
-            if (k < nc) acc[k] = fmaf(ylds[j][k], x, acc[k]);
+          for (int k = 0; k < KPT; ++k) acc[k] = fmaf(ylds[j * kTmRow + k0 + k], x, acc[k]);
         }
       }
     }
   }
-  if (t < cols) {
+  if (live) {
     float *o = a.transfer + (size_t)(a.v_begin + vl) * nc * cols;
 #pragma unroll
-    for (int k = 0; k < kShCoeffs; ++k)
-      if (k < nc) o[(size_t)k * cols + t] = acc[k];
+    for (int k = 0; k < KPT; ++k)
+      if (k0 + k < nc) o[(size_t)(k0 + k) * cols + col] = acc[k];
   }
 }
 
 }  // namespace
 
-size_t env_table_doubles(int n) { return kTabHead + 6 * env_face_doubles(n); }
+size_t env_table_doubles(int n) { return table_doubles(n); }
 
-void launch_env_tables(const float *faces, int n, double *tab, hipStream_t s) {
-  require(faces && tab && n >= 1 && n <= 128, NWPRT_ERR_INVALID_ARGUMENT,
+void launch_env_tables(const float *faces, int n, int maps, double *tab, hipStream_t s) {
+  require(faces && tab && n >= 1 && n <= 128 && maps >= 1, NWPRT_ERR_INVALID_ARGUMENT,
           "env tables: face size must be in [1, 128]");
-  hipLaunchKernelGGL(env_rows_kernel, dim3(6 * n), dim3(128), 0, s, faces, n, tab);
+  hipLaunchKernelGGL(env_rows_kernel, dim3(6 * n, maps), dim3(128), 0, s, faces, n, tab);
   hip_check(hipGetLastError(), "env_rows_kernel launch");
-  hipLaunchKernelGGL(env_marginals_kernel, dim3(6), dim3(128), 0, s, n, tab);
+  hipLaunchKernelGGL(env_marginals_kernel, dim3(6, maps), dim3(128), 0, s, n, tab);
   hip_check(hipGetLastError(), "env_marginals_kernel launch");
-  hipLaunchKernelGGL(env_face_table_kernel, dim3(1), dim3(64), 0, s, tab);
+  hipLaunchKernelGGL(env_face_table_kernel, dim3(maps), dim3(64), 0, s, n, tab);
   hip_check(hipGetLastError(), "env_face_table_kernel launch");
 }
 
@@ -1806,8 +1831,7 @@ void launch_sh_render(const ShArgs &a, hipStream_t s) {
   require(a.degree >= 0 && a.degree <= kShMaxDegree && a.samples >= 1 && a.width > 0 &&
               a.height > 0 && a.n_tris > 0 && a.n_vertices > 0,
           NWPRT_ERR_INVALID_ARGUMENT, "sh_render: bad degree, sample count or size");
-  hipLaunchKernelGGL(sh_light_response_kernel, dim3((unsigned)((a.n_vertices + 3) / 4)),
-                     dim3(256), 0, s, a);
+  hipLaunchKernelGGL(sh_light_response_kernel, dim3((unsigned)a.n_vertices), dim3(256), 0, s, a);
   hip_check(hipGetLastError(), "sh_light_response_kernel launch");
   constexpr int pairs_per_block = 64 / kShPairLanes;
   const dim3 corner_grid((unsigned)((a.n_keys + pairs_per_block - 1) / pairs_per_block));
@@ -1852,7 +1876,12 @@ void launch_sh_transfer(const TmArgs &a, hipStream_t s) {
   else
     hipLaunchKernelGGL(tm_light_kernel<false>, light_grid, dim3(64), 0, s, a);
   hip_check(hipGetLastError(), "tm_light_kernel launch");
-  hipLaunchKernelGGL(tm_project_kernel, dim3((unsigned)a.n_verts), dim3(256), 0, s, a);
+  // 256 threads hold nc rows of 3 nc columns at 9 rows a thread up to degree 4
+  // (25 rows of 75 columns), at 27 at degree 5, at all rows above.
+  const dim3 pgrid((unsigned)a.n_verts);
+  if (a.degree <= 4) hipLaunchKernelGGL((tm_project_kernel<9, 32>), pgrid, dim3(256), 0, s, a);
+  else if (a.degree <= 5) hipLaunchKernelGGL((tm_project_kernel<27, 16>), pgrid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((tm_project_kernel<kShCoeffs, 16>), pgrid, dim3(256), 0, s, a);
   hip_check(hipGetLastError(), "tm_project_kernel launch");
 }
 

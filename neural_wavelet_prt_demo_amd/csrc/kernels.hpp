@@ -233,9 +233,10 @@ struct CastArgs {
 };
 // Doubles of the environment sampling tables for face size n: face pmf[6],
 // face cdf[7], then per face cdf_rows[n][n+1], pdf_rows[n][n],
-// cdf_marginals[n+1], pdf_marginals[n].
+// cdf_marginals[n+1], pdf_marginals[n].  launch_env_tables builds those of
+// `maps` maps, the faces and the tables each one after the other.
 size_t env_table_doubles(int n);
-void launch_env_tables(const float *faces, int n, double *tab, hipStream_t s);
+void launch_env_tables(const float *faces, int n, int maps, double *tab, hipStream_t s);
 void launch_gbuffer_cast(const CastArgs &a, hipStream_t s);
 
 // SH-PRT render (gbuffer_kernels.hip): per-vertex light response, colour

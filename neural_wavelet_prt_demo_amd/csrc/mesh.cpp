@@ -563,7 +563,7 @@ nwprt_status nwprt_gbuffer_cast(nwprt_ctx ctx, int32_t mesh_id, const nwprt_came
               NWPRT_ERR_INVALID_ARGUMENT, "gbuffer_cast: direct_samples must be in [1, 2^20]");
       check_aligned(gbuffer->direct, 16, "G-buffer direct");
       ctx->env_tables.ensure(env_table_doubles(params->light_env_n) * sizeof(double));
-      launch_env_tables(params->light_env_faces, params->light_env_n,
+      launch_env_tables(params->light_env_faces, params->light_env_n, 1,
                         ctx->env_tables.as<double>(), pick(ctx, stream));
       a.light_faces = params->light_env_faces;
       a.env_tab = ctx->env_tables.as<double>();
@@ -670,11 +670,9 @@ nwprt_status nwprt_sh_compute_transfer(nwprt_ctx ctx, int32_t mesh_id, const flo
     if (vertex_count == 0) return;
     const hipStream_t st = pick(ctx, stream);
     const int nc = (degree + 1) * (degree + 1);
-    const size_t td = env_table_doubles(face_n), face_floats = (size_t)6 * face_n * face_n * 3;
+    const size_t td = env_table_doubles(face_n);
     ctx->sh_tables.ensure(td * nc * sizeof(double));
-    for (int i = 0; i < nc; ++i)
-      launch_env_tables(basis_faces + face_floats * i, face_n, ctx->sh_tables.as<double>() + td * i,
-                        st);
+    launch_env_tables(basis_faces, face_n, nc, ctx->sh_tables.as<double>(), st);
     // Vertices per launch: the path records, start-direction bases and
     // per-(sample, map) radiance of a launch stay within kTmWorkBudget, and
     // the (vertex, sample, map) triples within one grid.

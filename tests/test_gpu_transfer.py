@@ -91,6 +91,21 @@ def test_transfer_replays_oracle(nw, orc, ctx, deg, samples, max_bounce, disney)
     ctx.mesh_destroy(mesh)
 
 
+@pytest.mark.parametrize("deg,samples", [(0, 1), (3, 33), (4, 31), (5, 17), (6, 16), (7, 15)])
+def test_transfer_projection_tiles(nw, orc, ctx, deg, samples):
+    """Rows and columns of the projection at every split over a workgroup's
+    threads, with samples around its chunks of 32 and 16."""
+    v, ix, mids, mats, pts = panel_scene()
+    pts = pts[::4]
+    basis = smooth_basis((deg + 1) ** 2, seed=deg)
+    mesh = _mesh(ctx, v, ix, mats, mids)
+    got = _transfer(nw, ctx, mesh, basis, deg, len(v), samples=samples, seed=3)
+    ref = orc.sh_transfer(v, ix, mats, basis, deg, material_ids=mids, samples=samples, seed=3,
+                          verts=pts)
+    _compare(got[pts], ref, f"deg {deg} samples {samples}")
+    ctx.mesh_destroy(mesh)
+
+
 def test_transfer_with_vertex_normals_replays_oracle(nw, orc, ctx):
     """Smooth-shaded geometry: a faceted bowl (interpolated normals differ
     from the geometric ones) with a floor; degree 2, 384 samples."""
