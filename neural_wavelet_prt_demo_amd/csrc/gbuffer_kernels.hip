@@ -66,6 +66,7 @@ __device__ inline bool box_entry(float3 lo, float3 hi, float3 o, float3 inv, flo
 // triangle test by the lanes at a leaf; `node` is the lane's node (>= 0), its
 // leaf reference (< 0: the triangles of ~node not tested yet) or kDone.
 constexpr int kDone = INT_MIN;
+constexpr int kStackRows = kBvhMaxDepth + 1;
 
 // Sums of products with every rounding written out, so that each kernel that
 // traces a ray finds the same hits bit for bit.
@@ -83,62 +84,67 @@ __device__ inline float dot_yxz(float3 a, float3 b) {
 }
 
 // Triangle ~node >> 3 against the ray, then the lane's next triangle or entry.
+// Without branches: some lane of a wave nearly always passes each test, and the
+// hit's registers need no copies (transfer matrices of 2116 vertices, 64
+// samples, degree 4, whole call: 2.96 -> 2.84 ms with node_step's).
 template <bool ANY>
 __device__ inline void leaf_step(const BvhTri *__restrict__ tris, float3 o, float3 d, int *stack,
                                  int &node, int &sp, Hit &h) {
 #pragma clang fp contract(off)
   const int ref = ~node, slot = ref >> 3;
-  const float4 *r = reinterpret_cast<const float4 *>(tris + slot);
+  // slot < 2^28, so the offset in float4s fits 32 bits.
+  const float4 *r = reinterpret_cast<const float4 *>(tris) + (uint32_t)(3 * slot);
   const float4 a = r[0], b = r[1], c = r[2];
-  if (ref & 7) node = ~(ref + 7);  // first + 1, count - 1
-  else node = sp == 0 ? kDone : stack[64 * --sp];
   const float3 e1 = v3(b), e2 = v3(c);
   const float3 p = cross_fma(d, e2);
   const float det = dot_yxz(e1, p);
-  if (det == 0.0f) return;
   const float inv = 1.0f / det;
   const float3 s = sub(o, v3(a));
   const float u = dot_xyz(s, p) * inv;
-  if (!(u >= 0.0f && u <= 1.0f)) return;
   const float3 q = cross_fma(s, e1);
   const float dq = dot_yxz(d, q), v = dq * inv;
-  if (!(v >= 0.0f && fmaf(dq, inv, u) <= 1.0f)) return;
   const float t = dot_yxz(e2, q) * inv;
   const int prim = __float_as_int(a.w);
-  if (t > kTmin && (t < h.t || (t == h.t && prim < h.prim))) {
-    h = Hit{t, u, v, prim, slot};
-    if (ANY) node = kDone;
-  }
+  const bool hit = (det != 0.0f) & (u >= 0.0f) & (u <= 1.0f) & (v >= 0.0f) &
+                   (fmaf(dq, inv, u) <= 1.0f) & (t > kTmin) &
+                   ((t < h.t) | ((t == h.t) & (prim < h.prim)));
+  h.t = hit ? t : h.t;
+  h.u = hit ? u : h.u;
+  h.v = hit ? v : h.v;
+  h.prim = hit ? prim : h.prim;
+  h.slot = hit ? slot : h.slot;
+  const bool last = (ref & 7) == 0;
+  node = ANY && hit ? kDone : ~(ref + 7);  // first + 1, count - 1
+  if (last && !(ANY && hit)) node = stack[64 * --sp];
 }
 
 // Both children's boxes of internal node `node`: on to the nearer one that is
-// hit (ANY: the first), the other pushed, or to the top of the stack.  The
-// host bounds the tree at kBvhMaxDepth internal levels and a path pushes at
-// most one entry per level, so sp stays within the bound.
+// hit (ANY: the first), the other pushed, or to the top of the stack, whose
+// lowest entry is kDone.  The host bounds the tree at kBvhMaxDepth internal
+// levels and a path pushes at most one entry per level, so a node of internal
+// level l < kBvhMaxDepth is met with at most l entries above that one, and the
+// slot above them (taken only by a lane that pushes) lies within kStackRows.
 template <bool ANY>
 __device__ inline void node_step(const BvhNode *__restrict__ nodes, float3 o, float3 inv,
                                  float tmax, int *stack, int &node, int &sp) {
   const float4 *nr = reinterpret_cast<const float4 *>(nodes + node);
   const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2], n3 = nr[3];
-  int c0 = __float_as_int(n0.w), c1 = __float_as_int(n1.w);
+  const int c0 = __float_as_int(n0.w), c1 = __float_as_int(n1.w);
   float t0, t1;
   const bool h0 = box_entry(v3(n0), v3(n1), o, inv, tmax, t0);
   const bool h1 = box_entry(v3(n2), v3(n3), o, inv, tmax, t1);
-  if (h0 && h1) {
-    if (!ANY && t1 < t0) {
-      const int c = c0;
-      c0 = c1;
-      c1 = c;
-    }
-    if (sp < kBvhMaxDepth) stack[64 * sp++] = c1;
-    node = c0;
-  } else if (h0) {
-    node = c0;
-  } else if (h1) {
-    node = c1;
-  } else {
-    node = sp == 0 ? kDone : stack[64 * --sp];
-  }
+  const bool second = ANY ? !h0 : !h0 | (h1 & (t1 < t0));  // c1 is next
+  stack[64 * sp] = second ? c0 : c1;
+  sp += h0 & h1;
+  node = second ? c1 : c0;
+  if (!(h0 | h1)) node = stack[64 * --sp];
+}
+
+// A fresh walk: the root, and the entry that ends it.
+__device__ inline void walk_begin(int *stack, int &node, int &sp) {
+  stack[0] = kDone;
+  node = 0;
+  sp = 1;
 }
 
 // The walk of a wave's rays.  Bound: dependent node and triangle fetches, and
@@ -157,7 +163,8 @@ __device__ inline Hit walk(const BvhNode *__restrict__ nodes, const BvhTri *__re
   Hit h{kTmax, 0.0f, 0.0f, INT_MAX, 0};
   auto safe_inv = [](float x) { return 1.0f / (fabsf(x) > 1e-30f ? x : copysignf(1e-30f, x)); };
   const float3 inv = v3(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
-  int node = 0, sp = 0;
+  int node, sp;
+  walk_begin(stack, node, sp);
   for (;;) {
     const int inner = __popcll(__ballot(node >= 0));
     const int leaf = __popcll(__ballot(node < 0 && node != kDone));
@@ -172,7 +179,7 @@ __device__ inline Hit walk(const BvhNode *__restrict__ nodes, const BvhTri *__re
 }
 
 // Closest hit along o + t d, t in (kTmin, kTmax).  stack points at this
-// lane's column of a [kBvhMaxDepth][64] LDS array.
+// lane's column of a [kStackRows][64] LDS array.
 __device__ inline Hit trace(const BvhNode *__restrict__ nodes, const BvhTri *__restrict__ tris,
                             float3 o, float3 d, int *stack) {
   return walk<false>(nodes, tris, o, d, stack);
@@ -1053,7 +1060,7 @@ __global__ void env_face_table_kernel(int n, double *__restrict__ tab) {
 template <bool DIRECT, bool DS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void gbuffer_cast_kernel(
     CastArgs a) {
-  __shared__ int stack_lds[kBvhMaxDepth * 64];
+  __shared__ int stack_lds[kStackRows * 64];
   const int lane = threadIdx.x;
   const int tiles_x = (a.width + 7) >> 3;
   const int ix = (int)(blockIdx.x % (unsigned)tiles_x) * 8 + (lane & 7);
@@ -1376,7 +1383,7 @@ __global__ __launch_bounds__(64) void sh_corner_kernel(ShArgs a) {
 // Per pixel: the primary ray's first hit interpolates its triangle's corner
 // colours; a miss shows the view environment (devicePrograms.cu:519-522).
 __global__ __launch_bounds__(64) void sh_pixel_kernel(ShArgs a) {
-  __shared__ int stack_lds[kBvhMaxDepth * 64];
+  __shared__ int stack_lds[kStackRows * 64];
   const int lane = threadIdx.x;
   const int tiles_x = (a.width + 7) >> 3;
   const int ix = (int)(blockIdx.x % (unsigned)tiles_x) * 8 + (lane & 7);
@@ -1506,8 +1513,8 @@ __device__ inline Surface tm_surface(const TmArgs &a, int mat, float3 ns, float3
 }
 
 template <bool DS>
-__global__ __launch_bounds__(64) void tm_paths_kernel(TmArgs a) {
-  __shared__ int stack_lds[kBvhMaxDepth * 64];
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void tm_paths_kernel(TmArgs a) {
+  __shared__ int stack_lds[kStackRows * 64];
   const int lane = threadIdx.x;
   const long long pair = (long long)blockIdx.x * 64 + lane;
   if (pair >= a.n_verts * a.samples) return;  // no barriers below
@@ -1638,7 +1645,7 @@ __device__ inline bool tm_nan3(float3 c) { return isnan(c.x) || isnan(c.y) || is
 
 template <bool DS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void tm_light_kernel(TmArgs a) {
-  __shared__ int stack_lds[kBvhMaxDepth * 64];
+  __shared__ int stack_lds[kStackRows * 64];
   const int lane = threadIdx.x;
   const int nc = (a.degree + 1) * (a.degree + 1);
   const long long q = (long long)blockIdx.x * 64 + lane;
