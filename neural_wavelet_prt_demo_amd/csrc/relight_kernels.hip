@@ -310,11 +310,9 @@ template <typename E, bool SP, int V>
 void launch_v(const RelightArgs &a, hipStream_t s) {
   constexpr MfmaVariant v = kMfmaVariants[V];
   if (a.aux) {
-    // Aux scenes are built for one tile shape, the pipelined one (1280 x 720, K =
-    // 64, FP16, both passes: 1232 us with two groups layer by layer, 1216 so),
-    // and variant 0's for the tap.
+    // Aux scenes are built for one tile shape (and variant 0's for the tap).
     if (a.dump) launch_shape<E, SP, true, true, 2, false, 2, false>(a, s);
-    else launch_shape<E, SP, false, true, 0, false, 2, true>(a, s);
+    else launch_shape<E, SP, false, true, 2, false, 2, true>(a, s);
   } else if (a.dump && V == 0) {
     launch_shape<E, SP, true, false, v.gp, v.w4_lds, v.min_waves, false>(a, s);
   } else {
