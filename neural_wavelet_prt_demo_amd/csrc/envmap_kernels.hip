@@ -229,6 +229,9 @@ __device__ void select_digit(const uint32_t *hist, uint32_t *wt, int shift, uint
 // - Keys above the chosen first-digit bucket are taken at once; keys in it
 //   (at most kTopkCand of them) move to LDS, and the remaining digits are
 //   resolved there.  A larger bucket falls back to passes over all keys.
+// Bound: the latency of one workgroup's loads, so the histograms are summed by
+// all threads and the scores read several 16 B loads ahead (6 x 128 x 128
+// scores, K = 300: one load at a time 52.7 us, so 22.6).
 constexpr int kTopkCand = 3072;
 constexpr int kScoreBlock = 256;
 
@@ -264,7 +267,7 @@ __global__ __launch_bounds__(kTopkBlock) void topk_kernel(const float *__restric
                                                           int n_wg,
                                                           int32_t *__restrict__ out_idx,
                                                           float *__restrict__ out_str) {
-  __shared__ uint32_t hist[256], wt[4];
+  __shared__ uint32_t hist[256], wt[4], part[kTopkBlock];
   __shared__ uint64_t sel[NWPRT_MAX_K], sorted[NWPRT_MAX_K];
   __shared__ uint64_t cand[kTopkCand];
   __shared__ uint64_t s_prefix, s_mask;
@@ -281,11 +284,15 @@ __global__ __launch_bounds__(kTopkBlock) void topk_kernel(const float *__restric
     s_count = 0;
     s_ncand = 0;
   }
-  if (tid < 256) {
+  {
     uint32_t h = 0;
-    for (int w = 0; w < n_wg; ++w) h += wg_hist[(size_t)w * 256 + tid];
-    hist[tid] = h;
+#pragma unroll 8
+    for (int w = tid >> 8; w < n_wg; w += kTopkBlock / 256)
+      h += wg_hist[(size_t)w * 256 + (tid & 255)];
+    part[tid] = h;
   }
+  __syncthreads();
+  if (tid < 256) hist[tid] = part[tid] + part[tid + 256] + part[tid + 512] + part[tid + 768];
   __syncthreads();
   select_digit(hist, wt, 56, &s_prefix, &s_mask, &s_need, &s_done);
   const uint32_t d1 = (uint32_t)(s_prefix >> 56);
@@ -308,14 +315,32 @@ __global__ __launch_bounds__(kTopkBlock) void topk_kernel(const float *__restric
     }
   };
   if (in_lds) {
-    for (int t = tid; t < M; t += kTopkBlock) {
-      const uint64_t key = topk_key(scores, t);
-      const uint32_t top = (uint32_t)(key >> 56);
-      if (top > d1) {
-        const uint32_t pos = atomicAdd(&s_count, 1u);
-        if (pos < (uint32_t)NWPRT_MAX_K) sel[pos] = key;
-      } else if (top == d1) {
-        cand[atomicAdd(&s_ncand, 1u)] = key;
+    // Four scores a load, kAhead loads in flight (M is a multiple of 4).
+    constexpr int kAhead = 6;
+    for (int q0 = tid; q0 < M / 4; q0 += kTopkBlock * kAhead) {
+      uint4 v[kAhead];
+#pragma unroll
+      for (int a = 0; a < kAhead; ++a) {
+        const int q = q0 + a * kTopkBlock;
+        v[a] = q < M / 4 ? ((const uint4 *)scores)[q] : make_uint4(0u, 0u, 0u, 0u);
+      }
+#pragma unroll
+      for (int a = 0; a < kAhead; ++a) {
+        const int q = q0 + a * kTopkBlock;
+        const uint32_t sc[4] = {v[a].x, v[a].y, v[a].z, v[a].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t top = sc[e] >> 24;
+          if (q >= M / 4 || top < d1) continue;
+          const uint64_t key =
+              ((uint64_t)sc[e] << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)(4 * q + e));
+          if (top > d1) {
+            const uint32_t pos = atomicAdd(&s_count, 1u);
+            if (pos < (uint32_t)NWPRT_MAX_K) sel[pos] = key;
+          } else {
+            cand[atomicAdd(&s_ncand, 1u)] = key;
+          }
+        }
       }
     }
     __syncthreads();
@@ -381,17 +406,27 @@ __global__ __launch_bounds__(256) void prepare_selection_kernel(
   if (planar && proj)
     for (int i = t; i < 32 * 32; i += 256) pj[i] = proj[i];
   __syncthreads();
-  // First-layer weight of output row m at contraction slot j: W1[m][j] w[j]
+  // First-layer weights of output row m at contraction slots j0 ..: W1[m][j] w[j]
   // for row-layout features; for planar ones the raw feature planar_feature(j)
-  // with the projection folded in, sum_i W1[m][i] w[i] P[i][f].
-  auto weight = [&](int m, int j) -> float {
-    if (!planar) return w1[m * 32 + j] * wk[j];
-    const int f = planar_feature(j);
-    if (!proj) return w1[m * 32 + f] * wk[f];
-    float acc = 0.0f;
+  // with the projection folded in, sum_i W1[m][i] w[i] P[i][f].  Eight slots at
+  // a time, so W1's row is read once for them (K = 300, both tile forms:
+  // 32 -> 9 us).
+  auto weights = [&](int m, int j0, float(&v)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int f = planar ? planar_feature(j0 + j) : j0 + j;
+      v[j] = planar && proj ? 0.0f : w1[m * 32 + f] * wk[f];
+    }
+    if (!(planar && proj)) return;
+    int f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = planar_feature(j0 + j);
 #pragma unroll 8
-    for (int i = 0; i < 32; ++i) acc = fmaf(w1[m * 32 + i] * wk[i], pj[i * 32 + f], acc);
-    return acc;
+    for (int i = 0; i < 32; ++i) {
+      const float x = w1[m * 32 + i] * wk[i];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = fmaf(x, pj[i * 32 + f[j]], v[j]);
+    }
   };
   if (mk32) {
     // 32x32x16 A operand: block b = t / 128 (rows 32 b + lane % 32), K step
@@ -399,8 +434,7 @@ __global__ __launch_bounds__(256) void prepare_selection_kernel(
     const int b = t >> 7, s = (t >> 6) & 1, lane = t & 63;
     const int m = 32 * b + (lane & 31);
     float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = weight(m, 16 * s + 8 * (lane >> 5) + j);
+    weights(m, 16 * s + 8 * (lane >> 5), v);
     dev::u32x4 out;
 #pragma unroll
     for (int d = 0; d < 4; ++d) out[d] = dev::pack_bf16(v[2 * d], v[2 * d + 1]);
@@ -410,8 +444,7 @@ __global__ __launch_bounds__(256) void prepare_selection_kernel(
     const int b = t >> 6, lane = t & 63, g = lane >> 4;
     const int m = 16 * b + (lane & 15);
     float v[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) v[s] = weight(m, 8 * g + s);
+    weights(m, 8 * g, v);
     dev::u32x4 out;
 #pragma unroll
     for (int d = 0; d < 4; ++d)

@@ -15,6 +15,7 @@
 // is in relight_mma16_device.hpp.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -183,12 +184,19 @@ __global__ __launch_bounds__(kRelightBlock) void calib_amax_kernel(RelightArgs a
     }
   const u32x4 *mk = (const u32x4 *)a.mk;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  u32x4 next[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) next[b] = mk[((size_t)k0 * 4 + b) * 64 + lane];
   float m[3] = {0.f, 0.f, 0.f};
   auto upd = [](float &mm, f32x4 c) { mm = fmaxf(mm, fmaxf(fmaxf(c[0], c[1]), fmaxf(c[2], c[3]))); };
   for (int k = k0; k < k1; ++k) {
     u32x4 a1[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) a1[b] = mk[((size_t)k * 4 + b) * 64 + lane];
+    for (int b = 0; b < 4; ++b) a1[b] = next[b];
+    if (k + 1 < k1) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) next[b] = mk[((size_t)(k + 1) * 4 + b) * 64 + lane];
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       f32x4 c[4];
@@ -218,7 +226,13 @@ __global__ __launch_bounds__(kRelightBlock) void calib_amax_kernel(RelightArgs a
     float v = m[i];
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-    if (lane == 0) atomicMax((unsigned int *)a.amax + i, __float_as_uint(v));
+    // The maxima only grow: a wave whose own is not above the one it reads
+    // has nothing to add (thousands of atomics on three words took most of
+    // this kernel's time).
+    unsigned int *at = (unsigned int *)a.amax + i;
+    if (lane == 0 && __float_as_uint(v) > __hip_atomic_load(at, __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(at, __float_as_uint(v));
   }
 }
 
@@ -257,8 +271,8 @@ __global__ __launch_bounds__(256) void calib_gather_kernel(const uint16_t *__res
   }
 }
 
-// The calibration subsample encoded from positions: thread q computes the 16
-// levels of frame pixel q * stride with the standalone planar encode's
+// The calibration subsample encoded from positions: thread q of plane r =
+// blockIdx.y computes levels r and 15 - r of frame pixel q * stride with the standalone planar encode's
 // arithmetic (plane r = levels r and 15 - r, each accumulated from zero) and
 // writes the planar layout [8][n_cal][4] in BF16; background pixels get
 // zeros.  Block 0 clears the four maxima.
@@ -266,8 +280,8 @@ template <bool HF16>
 __global__ __launch_bounds__(256) void calib_encode_kernel(RelightArgs a, int stride,
                                                            uint16_t *__restrict__ calib,
                                                            int n_cal, float *__restrict__ amax) {
-  if (blockIdx.x == 0 && threadIdx.x < 4) amax[threadIdx.x] = 0.f;
-  const int q = blockIdx.x * 256 + threadIdx.x;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 4) amax[threadIdx.x] = 0.f;
+  const int q = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
   if (q >= n_cal) return;
   const long long p = (long long)q * stride;
   const bool hit = p < a.n_pixels && (a.env_flag == nullptr || a.env_flag[p] != 0);
@@ -279,14 +293,12 @@ __global__ __launch_bounds__(256) void calib_encode_kernel(RelightArgs a, int st
     x[2] = x4.z;
   }
   uint2 *dst = (uint2 *)calib;
-  for (int r = 0; r < 8; ++r) {
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (hit) {
-      dev::accumulate_level<2, HF16>(a.lv, a.hash, r, x, v, nullptr);
-      dev::accumulate_level<2, HF16>(a.lv, a.hash, 15 - r, x, v + 2, nullptr);
-    }
-    dst[(size_t)r * n_cal + q] = make_uint2(dev::pack_bf16(v[0], v[1]), dev::pack_bf16(v[2], v[3]));
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  if (hit) {
+    dev::accumulate_level<2, HF16>(a.lv, a.hash, r, x, v, nullptr);
+    dev::accumulate_level<2, HF16>(a.lv, a.hash, 15 - r, x, v + 2, nullptr);
   }
+  dst[(size_t)r * n_cal + q] = make_uint2(dev::pack_bf16(v[0], v[1]), dev::pack_bf16(v[2], v[3]));
 }
 
 __global__ __launch_bounds__(256) void tonemap_kernel(const float *__restrict__ src,
@@ -481,7 +493,7 @@ void launch_calib_encode(const RelightArgs &enc, int stride, uint16_t *calib, in
               n_cal >= 1 && (long long)(n_cal - 1) * stride < enc.n_pixels &&
               enc.lv.n_levels == 16,
           NWPRT_ERR_INVALID_ARGUMENT, "calibration encode: bad subsample");
-  const dim3 grid((n_cal + 255) / 256);
+  const dim3 grid((n_cal + 255) / 256, 8);
   if (enc.hash_f16)
     hipLaunchKernelGGL(calib_encode_kernel<true>, grid, dim3(256), 0, s, enc, stride, calib, n_cal,
                        amax);
@@ -495,8 +507,13 @@ void launch_calibrate_amax(const RelightArgs &a, hipStream_t s) {
   require(a.n_pixels >= 1 && a.k >= 1 && a.k <= NWPRT_MAX_K && a.features && a.mk &&
               a.w_tiles && a.amax && (!a.aux || a.waux_tiles),
           NWPRT_ERR_INVALID_ARGUMENT, "calibration: missing operand");
-  constexpr int kChunk = 16;
-  const dim3 grid((a.n_pixels + kRelightBlock - 1) / kRelightBlock, (a.k + kChunk - 1) / kChunk);
+  // As many chunks of wavelets as make one round of the chip (256 CUs, three
+  // workgroups each): 16,384 pixels, K = 300: chunks of 16 (1.6 rounds, each
+  // step waiting for its tiles, each wave its atomics) 212 us, so 124.
+  constexpr int kRound = 768;
+  const int px = (a.n_pixels + kRelightBlock - 1) / kRelightBlock;
+  const int splits = std::min(a.k, std::max(1, kRound / px)), kChunk = (a.k + splits - 1) / splits;
+  const dim3 grid(px, (a.k + kChunk - 1) / kChunk);
   if (a.aux)
     hipLaunchKernelGGL(calib_amax_kernel<true>, grid, dim3(kRelightBlock), 0, s, a, kChunk);
   else
