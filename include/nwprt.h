@@ -711,7 +711,9 @@ nwprt_status nwprt_debug_hash_encode(nwprt_ctx ctx, int32_t scene_id,
                                      void *stream);
 /* Transport tap: per-pair network output T (after output activation) for
  * pixels [pixel_begin, pixel_begin + n_pixels) of a frame: device
- * float[n_pixels][K][3].  Uses the same kernels as nwprt_relight. */
+ * float[n_pixels][K][3].  Uses the same kernels as nwprt_relight.  Rows of
+ * background pixels (env_flag 0) hold nothing of use: FP32 leaves them
+ * untouched, the MFMA forms may write the network's output there. */
 nwprt_status nwprt_debug_transport(nwprt_ctx ctx, int32_t scene_id,
                                    int32_t env_id, const nwprt_gbuffer *gbuffer,
                                    int32_t width, int32_t height,

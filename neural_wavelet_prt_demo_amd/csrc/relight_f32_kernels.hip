@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kBlock) void relight_f32_kernel(RelightArgs a) {
           tr[ch] = a.softplus ? dev::softplus(acc) : acc;
           if (DUMP) {
             const int q = my_px - a.dump_begin;
-            if (mine && g < NG && q >= 0 && q < a.dump_count)
+            if (hit && g < NG && q >= 0 && q < a.dump_count)  // background rows stay
               a.dump[((size_t)q * a.k + k) * 3 + ch] = tr[ch];
           }
         }

@@ -41,3 +41,26 @@ def test_f32_shapes_agree_and_match_the_oracle(nw, orc, ctx, aux, k):
             assert np.array_equal(v.view(np.uint32), full[name][:p].view(np.uint32)), (p, name)
     ctx.envmap_destroy(env)
     ctx.scene_destroy(scene)
+
+
+@pytest.mark.parametrize("p", [1000, 20000, 65536 + 77])
+def test_f32_tap_leaves_background_rows(nw, orc, ctx, p):
+    """The transport tap of each launch shape writes the hit pixels' rows, as
+    the oracle has them, and no row of a background pixel (the wrapper clears
+    the buffer first), wherever hits and background share a wave."""
+    k = 3
+    case = make_case(nw, orc, seed=6, width=p, height=1, face_size=8, k=k, background=0.4,
+                     log2_hashmap_size=12)
+    scene = ctx.scene_create(case.desc, case.params)
+    env = ctx.envmap_from_faces(case.faces, k)
+    idx, st = ctx.envmap_selection(env)
+    frame = nw.DeviceFrame(p, 1, case.gbuf)
+    t = ctx.debug_transport(scene, env, frame, 0, p, nw.PREC_FP32)
+    hit = case.gbuf["env_flag"].reshape(-1) != 0
+    assert 0.5 < hit.mean() < 0.7
+    assert not np.any(t[~hit])
+    at = np.nonzero(hit)[0][::max(1, p // 50)].astype(np.int32)
+    _, _, ref = case.oscene.relight(idx, st, case.gbuf, pixels=at, transport=True)
+    assert max_rel_err(ref.reshape(-1, 3), t[at].reshape(-1, 3)) <= TOL_FP32
+    ctx.envmap_destroy(env)
+    ctx.scene_destroy(scene)
