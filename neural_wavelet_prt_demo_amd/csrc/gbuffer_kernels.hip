@@ -1241,12 +1241,13 @@ __device__ inline void sh_eval(float3 w, float (&y)[kShCoeffs]) {
   }
 }
 
-// R[v][k] = sum_j T[v][k][j] (x) L[j].  A workgroup per vertex, a quarter of
-// its nc rows a wave; a row's nc x 3 floats are read by the 64 lanes together
-// (coalesced) and multiplied by L flattened the same way, then reduced
-// across the wave per channel.  Bound: HBM (18.6 K vertices of degree 8, 1.47 GB:
-// 345 us with a vertex a wave, 2.3 rounds of the chip's waves, 323 us so split;
-// 4.5 TB/s, a large copy's rate is 5.0).
+// R[v][k] = sum_j T[v][k][j] (x) L[j].  WPV waves of a 256-thread workgroup
+// per vertex (1 or 4), a part of its nc rows each; a row's nc x 3 floats are
+// read by the 64 lanes together (coalesced) and multiplied by L flattened the
+// same way, then reduced across the wave per channel.  Rows are independent,
+// so both forms give the same bits.  Bound: HBM (18.6 K vertices of degree 8,
+// 1.47 GB: 4.7 TB/s at WPV = 4, a large copy's rate is 5.0) from degree 2 on,
+// the waves' count below.
 __device__ inline float wave_sum(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -1262,12 +1263,17 @@ constexpr int kShRowsInFlight = 4;
 static_assert((kShMaxDegree + 1) * (kShMaxDegree + 1) * 3 <= 64 * kShRowSlots,
               "a transfer-matrix row must fit the wave's load slots");
 
+template <int WPV>
 __global__ __launch_bounds__(256) void sh_light_response_kernel(ShArgs a) {
+  static_assert(WPV == 1 || WPV == 4, "a wave or the workgroup's four a vertex");
   const int nc = (a.degree + 1) * (a.degree + 1), row = nc * 3;
   const int lane = threadIdx.x & 63;
-  const long long v = blockIdx.x;
-  const int per = (nc + 3) / 4;  // rows a wave
-  const int kb = per * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ke = min(kb + per, nc);
+  const long long v =
+      WPV == 1 ? (long long)blockIdx.x * 4 + (threadIdx.x >> 6) : (long long)blockIdx.x;
+  if (v >= a.n_vertices) return;  // whole waves leave together; no barriers below
+  const int per = (nc + WPV - 1) / WPV;  // rows a wave
+  const int kb = WPV == 1 ? 0 : per * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ke = min(kb + per, nc);
   const float *t = a.transfer + (size_t)v * nc * row;
   float *o = a.light_response + (size_t)v * row;
   float l[kShRowSlots];
@@ -1838,7 +1844,19 @@ void launch_sh_render(const ShArgs &a, hipStream_t s) {
   require(a.degree >= 0 && a.degree <= kShMaxDegree && a.samples >= 1 && a.width > 0 &&
               a.height > 0 && a.n_tris > 0 && a.n_vertices > 0,
           NWPRT_ERR_INVALID_ARGUMENT, "sh_render: bad degree, sample count or size");
-  hipLaunchKernelGGL(sh_light_response_kernel, dim3((unsigned)a.n_vertices), dim3(256), 0, s, a);
+  // Four waves a vertex from degree 2 on (1 while there are fewer vertices
+  // than SIMDs), one below, where four would have a row or less each.  Whole
+  // calls with one wave, four waves a vertex: 100 vertices of degree 1 15.2,
+  // 13.8 us; 2000 of degree 2 18.6, 17.6; 18.6 K of degree 8 331, 309, of degree
+  // 1 27.8, 29.9; 400 K of degree 2 662, 662, of degree 1 301, 363, of degree 0
+  // 102, 213.  Past the grid of 2^32 - 1 threads that HIP takes, one as well.
+  constexpr long long kSplitVertices = 0xFFFFFFFFll / 256;
+  const int split_degree = a.n_vertices <= 1024 ? 1 : 2;
+  if (a.degree >= split_degree && a.n_vertices <= kSplitVertices)
+    hipLaunchKernelGGL(sh_light_response_kernel<4>, dim3((unsigned)a.n_vertices), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(sh_light_response_kernel<1>, dim3((unsigned)((a.n_vertices + 3) / 4)),
+                       dim3(256), 0, s, a);
   hip_check(hipGetLastError(), "sh_light_response_kernel launch");
   constexpr int pairs_per_block = 64 / kShPairLanes;
   const dim3 corner_grid((unsigned)((a.n_keys + pairs_per_block - 1) / pairs_per_block));

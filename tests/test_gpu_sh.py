@@ -65,6 +65,86 @@ def test_sh_render_replays_oracle(nw, orc, ctx, seed, w, h, degree, samples, kin
     ctx.mesh_destroy(mesh)
 
 
+@pytest.mark.parametrize("degree", [0, 1, 2, 3])
+def test_sh_light_response_forms(nw, orc, ctx, degree):
+    """Light response by one wave (degree 0) and four waves a vertex, with a
+    vertex count that is no multiple of four and rows no multiple of the
+    waves: the oracle's colours."""
+    s = _scene(5, sphere=(11, 7), soup=3)
+    nv, nc, w, h = len(s["vertices"]), (degree + 1) ** 2, 24, 16
+    assert nv % 4
+    rng = np.random.default_rng(degree)
+    T = rng.normal(0, 0.5, (nv, nc, nc, 3)).astype(np.float32)
+    L = rng.normal(0, 1, (nc, 3)).astype(np.float32)
+    mesh = ctx.mesh_create(s["vertices"], s["indices"], s["materials"], normals=s["normals"],
+                           material_ids=s["material_ids"])
+    out = nw.DeviceBuffer(w * h * 16)
+    ctx.sh_render(mesh, np.reshape(s["camera"], (3, 3)), w, h, nw.DeviceBuffer.from_array(T),
+                  nw.DeviceBuffer.from_array(L), degree, out, brdf_samples=8, seed=5)
+    ctx.sync()
+    got = out.download(np.float32, (w * h, 4)).astype(np.float64)
+    want = orc.sh_render(s["vertices"], s["indices"], s["normals"], s["materials"], s["camera"],
+                         w, h, T, L, degree, material_ids=s["material_ids"], samples=8, seed=5)
+    safe = want["margin"] >= 1e-4
+    ref = want["color"][safe, :3]
+    err = np.abs(got[safe, :3] - ref) / (np.abs(ref) + 1e-2 * np.abs(ref).max())
+    assert err.max() <= 1e-3, err.max()
+    ctx.mesh_destroy(mesh)
+
+
+@pytest.mark.parametrize("degree,at_end", [(0, True), (2, False)])
+def test_sh_render_many_vertices(nw, orc, ctx, degree, at_end):
+    """More vertices than a launch of one 256-thread workgroup each could take
+    (2^32 threads): the render still runs, with a few of them in use (the last
+    ones at degree 0, the first at degree 2)."""
+    s = _scene(7, sphere=(16, 8), soup=4)
+    used, n, nc, w, h = len(s["vertices"]), (1 << 24) + 5, (degree + 1) ** 2, 24, 16
+    rng = np.random.default_rng(2)
+    T = rng.normal(0, 1, (used, nc, nc, 3)).astype(np.float32)
+    L = rng.normal(0, 1, (nc, 3)).astype(np.float32)
+    first = n - used if at_end else 0
+    v = np.zeros((n, 3), np.float32)
+    nr = np.zeros((n, 3), np.float32)
+    nr[:, 2] = 1.0
+    v[first:first + used], nr[first:first + used] = s["vertices"], s["normals"]
+    ix = s["indices"] + np.int32(first)
+    dT = nw.DeviceBuffer(n * nc * nc * 12)
+    if at_end:
+        full = np.zeros((n, nc, nc, 3), np.float32)
+        full[first:] = T
+        dT.upload(full)
+    else:
+        full = None
+        dT.zero()
+        dT.upload(T)
+    print(f"sh_render {n} vertices degree {degree}", flush=True)
+    mesh = ctx.mesh_create(v, ix, s["materials"], normals=nr, material_ids=s["material_ids"])
+    out = nw.DeviceBuffer(w * h * 16)
+    ctx.sh_render(mesh, np.reshape(s["camera"], (3, 3)), w, h, dT, nw.DeviceBuffer.from_array(L),
+                  degree, out, brdf_samples=8, seed=9)
+    ctx.sync()
+    got = out.download(np.float32, (w * h, 4))
+    ctx.mesh_destroy(mesh)
+    if at_end:
+        want = orc.sh_render(v, ix, nr, s["materials"], s["camera"], w, h, full, L, degree,
+                             material_ids=s["material_ids"], samples=8, seed=9)
+        safe = want["margin"] >= 1e-4
+        ref = want["color"][safe, :3]
+        err = np.abs(got[safe, :3] - ref) / (np.abs(ref) + 1e-2 * np.abs(ref).max())
+        assert err.max() <= 1e-3, err.max()
+    else:  # the same vertices alone, where four waves share each
+        mesh = ctx.mesh_create(v[:used], ix, s["materials"], normals=nr[:used],
+                               material_ids=s["material_ids"])
+        small = nw.DeviceBuffer(w * h * 16)
+        ctx.sh_render(mesh, np.reshape(s["camera"], (3, 3)), w, h, dT,
+                      nw.DeviceBuffer.from_array(L), degree, small, brdf_samples=8, seed=9)
+        ctx.sync()
+        ref = small.download(np.float32, (w * h, 4))
+        ctx.mesh_destroy(mesh)
+        assert np.any(ref[:, :3] != ref[0, :3])
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
 def test_sh_render_errors(nw, ctx):
     s = mesh_scene(0)  # has a mirror
     T = nw.DeviceBuffer(len(s["vertices"]) * 9 * 9 * 12)
