@@ -331,14 +331,16 @@ std::tuple<int, int, int> tune_key(nwprt_precision prec, int k, int n_pixels) {
 }
 
 // Kernel variant for a relight: the forced one (BF16 / FP16 only), else the
-// autotuner's choice for this shape bucket, else the form's default.
-int pick_variant(nwprt_ctx ctx, nwprt_precision prec, int k, int n_pixels) {
+// autotuner's choice for this shape bucket, else the form's default (that of
+// a relight which encodes its own pixels unless `fused` is false).
+int pick_variant(nwprt_ctx ctx, nwprt_precision prec, int k, int n_pixels, bool fused = true) {
   if (ctx->forced_variant >= 0 &&
       (prec != NWPRT_PREC_FP8 || ctx->forced_variant < relight_fp8_variant_count()))
     return ctx->forced_variant;
   auto it = ctx->tuned.find(tune_key(prec, k, n_pixels));
   if (it != ctx->tuned.end()) return it->second;
-  return prec == NWPRT_PREC_FP8 ? kDefaultFp8Variant : kDefaultMfmaVariant;
+  return prec == NWPRT_PREC_FP8 ? kDefaultFp8Variant
+                                : relight_mfma_default_variant(k, n_pixels, fused);
 }
 
 int variant_count(nwprt_precision prec) {
@@ -425,7 +427,8 @@ void relight_with(nwprt_ctx ctx, const Scene &sc, EnvMap &env, const nwprt_gbuff
                              scene_projection(sc));
     a.mk = w.mk;
     a.w_tiles = elem == Elem::BF16 ? sc.tiles_bf16.as<uint16_t>() : sc.tiles_f16.as<uint16_t>();
-    launch_relight_mfma(a, elem, variant >= 0 ? variant : pick_variant(ctx, prec, env.k, P), s);
+    launch_relight_mfma(a, elem,
+                        variant >= 0 ? variant : pick_variant(ctx, prec, env.k, P, fused), s);
   }
   hip_check(hipEventRecord(env.last_use, s), "hipEventRecord");
 }
@@ -468,8 +471,6 @@ void relight_from_slot(nwprt_ctx ctx, Scene &sc, int scene_id, EnvMap &env, Fram
 }
 
 // ------------------------------------------------------------------ batch --
-
-constexpr int kDefaultBatchVariant = 5;  // pipe.w4reg.occ2
 
 Batch &get_batch(nwprt_ctx ctx, int id) {
   auto it = ctx->batches.find(id);
@@ -679,7 +680,7 @@ void create_batch(nwprt_ctx ctx, const nwprt_batch_job *jobs, int n, nwprt_preci
   // each launch makes its stream wait for them.
   for (int j = 0; j < n; ++j)
     hip_check(hipEventSynchronize(get_env(ctx, b->jobs[j].env_id).ready), "hipEventSynchronize");
-  capture_batch(ctx, *b, fp8 ? kDefaultFp8Variant : kDefaultBatchVariant);
+  capture_batch(ctx, *b, fp8 ? kDefaultFp8Variant : kDefaultMfmaVariant);
   const int id = ctx->next_id++;
   ctx->batches[id] = std::move(b);
   *batch_id = id;

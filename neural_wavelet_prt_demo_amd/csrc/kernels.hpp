@@ -138,7 +138,10 @@ struct RelightArgs {
   nwprt_hashgrid_levels lv;
 };
 // Tile-shape variants of the fused kernel (see relight_kernels.hip).
-constexpr int kDefaultMfmaVariant = 5;  // pipe.w4reg.occ2
+constexpr int kDefaultMfmaVariant = 5;  // pipe.w4reg.occ2 (batches and servers, most relights)
+constexpr int kFewWaveletsVariant = 0;  // gp2.w4reg.occ2
+// One relight's, when none is tuned (fused: it encodes its own pixels).
+int relight_mfma_default_variant(int k, int n_pixels, bool fused);
 int relight_mfma_variant_count();
 const char *relight_mfma_variant_name(int variant);
 void launch_relight_mfma(const RelightArgs &a, Elem elem, int variant, hipStream_t s);

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -56,17 +57,40 @@ constexpr int kNumMfmaVariants = sizeof(kMfmaVariants) / sizeof(kMfmaVariants[0]
 // Workgroups that take 256 pixels (64 a wave) before the ones that take 64
 // together (relight_group).  The chip holds 512 workgroups of these kernels
 // (256 CUs, two waves a SIMD).  Whole rounds of 512 go 64 pixels a wave; the
-// rest of the frame, at most one round, is split finer unless it fills more
-// than three quarters of a round, where the finer form's four quarter rounds
-// would take longer than the one it replaces.  Measured, whole requests: 128 x
-// 128, K = 64, BF16 (64 workgroups before, 256 now) 142 -> 73 us; 1283 x 717,
-// K = 128, FP16 (7.02 rounds) 1875 -> 1705 us, half of it the pipelined step
-// becoming the untuned default (1920 x 1080, K = 300: 9423 -> 9145 us).
+// rest of the frame, at most one round, is split finer where that is shorter.
+// Unsplit it takes one time up to 256 workgroups (one a CU) and another up to
+// 512; split, a time that grows with its pixels and, as the four waves load
+// the weights and encode for a quarter of the wavelets each, has less to give
+// at small K.  Behind whole rounds it gains less, because the waves that finish
+// them early overlap with an unsplit rest too.  So each step of the rest has a
+// least K, between where the split is the shorter one along a surface (real
+// frames) and at scattered positions (every gather a line of its own); there
+// it is not above the two-group step without a split by more than 1.5 %.  BF16,
+// whole calls in us, unsplit / split (rounds + workgroups of the rest):
+//                     scattered   surface                   scattered   surface
+//   0 + 128, K =  8    48 /  40   37 / 26   1 + 192, K = 16  129 / 133   92 /  87
+//   0 + 192, K = 16    57 /  58   45 / 38   1 + 320, K =  8  149 / 150   92 /  83
+//   0 + 256, K = 32    74 /  83   61 / 57   1 + 384, K = 24  182 / 190  142 / 129
+//   0 + 320, K =  8    76 /  84   51 / 46   2 +  64, K = 48  303 / 274  255 / 228
+//   0 + 384, K = 24   100 / 108   76 / 67   4 + 192, K = 48  534 / 537  452 / 450
+//   1 + 128, K = 16   126 / 120   91 / 80   4 + 320, K = 24  414 / 417  335 / 317
+//   1 + 256, K = 64   241 / 256  209 / 214  4 + 384, K = 48  586 / 592  496 / 488
+// Features read from memory (p1 / p2, aux) leave only the weights' loads to
+// share, so those relights take the first lines behind any number of rounds
+// (aux: 0 + 128, K = 1 38.3 / 38.8, 4 0.94 of the time unsplit; 0 + 256, K = 24
+// 71.0 / 68.5; 3 + 320, K = 8 328 / 329, 64 0.95).
 constexpr int kRoundWgs = 512;
-int full_workgroups(int n_pixels) {
+int full_workgroups(int n_pixels, int k, bool fused) {
   const int wgs = (n_pixels + kRelightBlock - 1) / kRelightBlock;
-  const int rest = wgs % kRoundWgs;
-  return 4 * rest > 3 * kRoundWgs ? wgs : wgs - rest;
+  const int rest = wgs % kRoundWgs, rounds = wgs / kRoundWgs;
+  const bool behind = fused && rounds >= 2;
+  int least_k = INT_MAX;
+  if (rest <= 128) least_k = fused ? 1 : 4;
+  else if (rest <= 192) least_k = behind ? 40 : 16;
+  else if (rest <= 256) least_k = rounds >= 1 ? INT_MAX : fused ? 32 : 16;
+  else if (rest <= 320) least_k = behind ? 24 : 8;
+  else if (rest <= 384) least_k = behind ? 40 : 24;
+  return k >= least_k ? wgs - rest : wgs;
 }
 
 // Grid: `full` workgroups of 4 waves x 64 pixels -- wave w of the one with
@@ -84,7 +108,19 @@ __global__ __launch_bounds__(kRelightBlock, MINW) void relight_mfma_kernel(Relig
   if (SPLIT && (int)blockIdx.x >= full) {
     const int tail = (int)gridDim.x - full;
     const int base = full * kRelightBlock + dev::xcd_tile((int)blockIdx.x - full, tail) * 64;
-    relight_group<E, SOFTPLUS, AUX, !AUX>(a, base, wave, lane, feat_lds);
+    if constexpr (AUX) {
+      relight_group<E, SOFTPLUS, AUX, !AUX>(a, base, wave, lane, feat_lds);
+    } else {
+      // The arguments through a pointer of their own: relight_group takes
+      // levels by a run-time number, and seen as the same object that makes the
+      // compiler read the level parameters of the other workgroups' encode a
+      // dword at a time too (BF16, 12 rounds and 64 workgroups, scattered
+      // positions, whole calls: K = 32 1179 us, so 1116).
+      using Args = const RelightArgs __attribute__((address_space(4)));
+      Args *args = (Args *)__builtin_amdgcn_kernarg_segment_ptr();  // `a` is the first argument
+      asm volatile("" : "+s"(args));
+      relight_group<E, SOFTPLUS, AUX, !AUX>(*(const RelightArgs *)args, base, wave, lane, feat_lds);
+    }
     return;
   }
   if (W4LDS) {
@@ -96,6 +132,15 @@ __global__ __launch_bounds__(kRelightBlock, MINW) void relight_mfma_kernel(Relig
   if (base >= a.n_pixels) return;
   relight_wave<E, SOFTPLUS, DUMP, AUX, GP, W4LDS, !AUX>(a, base, lane, w4s,
                                                        feat_lds + (AUX ? 0 : wave * 64 * 16));
+}
+
+// Frames of less than a round that are split whole: sharing workgroups only.
+template <typename E, bool SOFTPLUS, bool AUX>
+__global__ __launch_bounds__(kRelightBlock, 2) void relight_group_kernel(RelightArgs a) {
+  __shared__ uint32_t lds[kGroupLdsWords];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  relight_group<E, SOFTPLUS, AUX, !AUX>(a, dev::xcd_tile(blockIdx.x, gridDim.x) * 64, wave, lane,
+                                        lds);
 }
 
 // Persistent batch form: a machine-sized grid whose waves take work items
@@ -309,13 +354,28 @@ __global__ __launch_bounds__(256) void tonemap_kernel(const float *__restrict__ 
   dst[p] = dev::tonemap_rgba8(v.x, v.y, v.z);
 }
 
-template <typename E, bool SP, bool DUMP, bool AUX, int GP, bool W4LDS, int MINW, bool SPLIT>
+// MAY_SPLIT: the rest of the frame may go to sharing workgroups.  A frame of
+// which nothing is split takes the instance without them, whose registers are
+// its own.
+template <typename E, bool SP, bool DUMP, bool AUX, int GP, bool W4LDS, int MINW, bool MAY_SPLIT>
 void launch_shape(const RelightArgs &a, hipStream_t s) {
   const int wgs = (a.n_pixels + kRelightBlock - 1) / kRelightBlock;
-  const int full = SPLIT ? full_workgroups(a.n_pixels) : wgs;
-  const int rest = full < wgs ? a.n_pixels - full * kRelightBlock : 0;
-  hipLaunchKernelGGL((relight_mfma_kernel<E, SP, DUMP, AUX, GP, W4LDS, MINW, SPLIT>),
-                     dim3(full + (rest + 63) / 64), dim3(kRelightBlock), 0, s, a, full);
+  if constexpr (MAY_SPLIT) {
+    const int full = full_workgroups(a.n_pixels, a.k, a.fused_encode != 0);
+    if (full == 0) {
+      hipLaunchKernelGGL((relight_group_kernel<E, SP, AUX>), dim3((a.n_pixels + 63) / 64),
+                         dim3(kRelightBlock), 0, s, a);
+      return;
+    }
+    if (full < wgs) {
+      const int rest = a.n_pixels - full * kRelightBlock;
+      hipLaunchKernelGGL((relight_mfma_kernel<E, SP, DUMP, AUX, GP, W4LDS, MINW, true>),
+                         dim3(full + (rest + 63) / 64), dim3(kRelightBlock), 0, s, a, full);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((relight_mfma_kernel<E, SP, DUMP, AUX, GP, W4LDS, MINW, false>), dim3(wgs),
+                     dim3(kRelightBlock), 0, s, a, wgs);
 }
 
 template <typename E, bool SP, int V>
@@ -328,13 +388,14 @@ void launch_v(const RelightArgs &a, hipStream_t s) {
   } else if (a.dump && V == 0) {
     launch_shape<E, SP, true, false, v.gp, v.w4_lds, v.min_waves, false>(a, s);
   } else {
-    launch_shape<E, SP, false, false, v.gp, v.w4_lds, v.min_waves, V == kDefaultMfmaVariant>(a, s);
+    launch_shape<E, SP, false, false, v.gp, v.w4_lds, v.min_waves,
+                 V == kDefaultMfmaVariant || V == kFewWaveletsVariant>(a, s);
   }
 }
 
 template <typename E, bool SP>
 void launch_sp(const RelightArgs &a, int variant, hipStream_t s) {
-  if (a.dump) variant = 0;  // the transport tap is built for the default variant only
+  if (a.dump) variant = 0;  // the transport tap is built for variant 0 only
   switch (variant) {
     case 0: launch_v<E, SP, 0>(a, s); break;
     case 1: launch_v<E, SP, 1>(a, s); break;
@@ -409,6 +470,19 @@ void build_weight_tiles(const float *w, Elem elem, std::vector<uint16_t> &out) {
 }
 
 int relight_mfma_variant_count() { return kNumMfmaVariants; }
+
+// The pipelined step is the faster one, except where the encode is fused and 8
+// to 27 wavelets follow it on frames of more than two rounds: each wave's
+// encode is then as long as its network, and the two-group step leaves the
+// encoding waves more room (BF16, 2432 workgroups, two-group / pipelined:
+// K = 8 333 / 354 us, 16 359 / 397, 24 407 / 416, 32 473 / 458, 64 748 / 718;
+// along a surface 222 / 218, 257 / 280, 315 / 336, 382 / 373; 896 workgroups:
+// 16 162 / 165, 24 183 / 182; p2 alone, 2496: 16 170 / 162).
+int relight_mfma_default_variant(int k, int n_pixels, bool fused) {
+  return fused && k >= 8 && k < 28 && n_pixels > 2 * kRoundWgs * kRelightBlock
+             ? kFewWaveletsVariant
+             : kDefaultMfmaVariant;
+}
 const char *relight_mfma_variant_name(int v) {
   return v >= 0 && v < kNumMfmaVariants ? kMfmaVariants[v].name : nullptr;
 }

@@ -43,7 +43,6 @@ constexpr int kTickItems = 1 << 16;   // work items per tick at most
 // larger tick delays no one, and every launch ends in a partly idle tail
 // (measured: 2^28 -> 2^30 lowers a lone request's latency by ~1 ms).
 constexpr int64_t kDefaultTickPairs = 1ll << 30;
-constexpr int kDefaultVariant = 5;    // pipe.w4reg.occ2
 
 double now_s() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
@@ -125,7 +124,7 @@ struct Tick {
 struct Server {
   nwprt_ctx ctx = nullptr;
   nwprt_server_config cfg{};
-  int variant = kDefaultVariant;
+  int variant = kDefaultMfmaVariant;
   hipStream_t prep = nullptr, launch = nullptr;
   bool softplus_set = false, softplus = true;
   Pool pool;
@@ -520,7 +519,7 @@ nwprt_status nwprt_server_create(nwprt_ctx ctx, const nwprt_server_config *confi
                 c.tonemap == NWPRT_TONEMAP_NONE,
             NWPRT_ERR_INVALID_ARGUMENT, "unknown tonemap source");
     const bool fp8 = c.precision == NWPRT_PREC_FP8;
-    const int variant = c.variant >= 0 ? c.variant : fp8 ? kDefaultFp8Variant : kDefaultVariant;
+    const int variant = c.variant >= 0 ? c.variant : fp8 ? kDefaultFp8Variant : kDefaultMfmaVariant;
     require(fp8 ? variant < relight_fp8_variant_count() : relight_batch_variant_ok(variant),
             NWPRT_ERR_INVALID_ARGUMENT, "server: tile variant has no persistent form");
     ServerPtr sv(new Server(), destroy_server);
