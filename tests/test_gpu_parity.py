@@ -68,6 +68,18 @@ def test_haar_many_maps_bit_exact(nw, orc, ctx, n, n_maps):
     assert e.value.status == nw.ERR_INVALID_ARGUMENT
 
 
+@pytest.mark.parametrize("n,k", [(8, 1), (8, 384), (16, 1), (16, 300), (16, 1024)])
+def test_topk_small_maps(nw, orc, ctx, n, k):
+    """Maps of a key or two a thread, the largest of them included, and K up
+    to every key of the map."""
+    faces = nw.synth_cubemap(n + k, n)
+    env = ctx.envmap_from_faces(faces, k)
+    idx, st = ctx.envmap_selection(env)
+    ridx, rst = orc.topk(orc.envmap_haar(faces), k)
+    assert np.array_equal(idx, ridx) and np.array_equal(st, rst.astype(np.float32))
+    ctx.envmap_destroy(env)
+
+
 def test_topk_ties_break_by_index(nw, orc, ctx):
     n = 16
     faces = np.ones((6, n, n, 3), np.float32)  # all DCs equal, all details 0
