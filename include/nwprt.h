@@ -361,7 +361,8 @@ nwprt_status nwprt_pass_p2(nwprt_ctx ctx, int32_t scene_id, int32_t env_id,
  * waves per SIMD).  nwprt_autotune_relight times every variant on one frame
  * and records the fastest for that (precision, K, pixel-count) bucket;
  * later relights falling in the bucket use it, others a default by K and
- * size (nwprt_selected_relight_variant names it).
+ * size (nwprt_selected_relight_variant names it).  Scenes with aux inputs
+ * have one tile shape: it is timed, and nothing is recorded.
  * The count and names below are those of the BF16 / FP16 kernel; the FP8
  * kernel has its own (nwprt_relight_fp8_variant_*), and autotuning or
  * querying with NWPRT_PREC_FP8 works on those. */

@@ -1057,13 +1057,18 @@ nwprt_status nwprt_autotune_relight(nwprt_ctx ctx, int32_t scene_id, int32_t env
       slot.valid = false;
     else
       encode_into(ctx, sc, scene_id, slot, gbuffer, width, height, elem, s);
+    // Scenes with aux inputs run one tile shape whatever the variant: it is
+    // timed, and the bucket is left to the scenes that have a choice.
+    const bool one_form = sc.desc.aux_dims != 0 && precision != NWPRT_PREC_FP8;
+    const int first = one_form ? kDefaultMfmaVariant : 0;
+    const int last = one_form ? first + 1 : variant_count(precision);
     hipEvent_t e0, e1;
     hip_check(hipEventCreate(&e0), "hipEventCreate");
     hip_check(hipEventCreate(&e1), "hipEventCreate");
-    int best = 0;
+    int best = first;
     float best_t = 0.f;
     try {
-      for (int v = 0; v < variant_count(precision); ++v) {
+      for (int v = first; v < last; ++v) {
         relight_from_slot(ctx, sc, scene_id, env, slot, gbuffer, width, height, nullptr,
                           precision, NWPRT_TONEMAP_NONE, s, nullptr, 0, 0, v, fused);
         float t = 0.f;
@@ -1077,7 +1082,7 @@ nwprt_status nwprt_autotune_relight(nwprt_ctx ctx, int32_t scene_id, int32_t env
           hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
           t = rep == 0 ? ms : std::min(t, ms);
         }
-        if (v == 0 || t < best_t) {
+        if (v == first || t < best_t) {
           best = v;
           best_t = t;
         }
@@ -1089,7 +1094,7 @@ nwprt_status nwprt_autotune_relight(nwprt_ctx ctx, int32_t scene_id, int32_t env
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    ctx->tuned[tune_key(precision, env.k, width * height)] = best;
+    if (!one_form) ctx->tuned[tune_key(precision, env.k, width * height)] = best;
     if (best_variant) *best_variant = best;
     if (best_ms) *best_ms = best_t;
   });

@@ -63,7 +63,8 @@ EDGES = [(0, 128, 1), (0, 129, 15), (0, 129, 16), (0, 192, 16), (0, 193, 31), (0
 
 
 @pytest.mark.parametrize("precision,softplus", [("bf16", True), ("fp16", False)])
-def test_split_rule_edges_same_bits(nw, orc, ctx, precision, softplus):
+def test_split_rule_edges_same_bits(nw, orc, precision, softplus):
+    ctx = nw.Context(0)  # nothing tuned
     p_max = max(512 * r + w for r, w, _ in EDGES) * 256
     case = make_case(nw, orc, seed=12, width=p_max, height=1, face_size=8, k=64, background=0.1,
                      log2_hashmap_size=12, softplus=softplus)
@@ -93,4 +94,26 @@ def test_split_rule_edges_same_bits(nw, orc, ctx, precision, softplus):
         err = max_rel_err(ref, a["indirect"][at, :3], floor=1e-3 if softplus else 1.0)
         assert err <= {"bf16": 2e-2, "fp16": 5e-3}[precision], (p, k)
         ctx.envmap_destroy(env)
-    ctx.scene_destroy(scene)
+    ctx.close()
+
+
+def test_autotune_on_aux_scene_leaves_the_bucket(nw, orc):
+    """Every variant of an aux scene is the same kernel, so tuning one names
+    the default and keeps what a scene with a choice recorded for the shape."""
+    w, h, k = 64, 48, 8
+    ctx = nw.Context(0)
+    scenes, frames = [], []
+    for aux in (False, True):
+        case = make_case(nw, orc, seed=3, width=w, height=h, face_size=8, k=k, aux=aux,
+                         log2_hashmap_size=12)
+        scenes.append(ctx.scene_create(case.desc, case.params))
+        frames.append(nw.DeviceFrame(w, h, case.gbuf))
+    env = ctx.envmap_from_faces(case.faces, k)
+    for prec in (nw.PREC_BF16, nw.PREC_FP16):
+        kept, _ = ctx.autotune_relight(scenes[0], env, frames[0], prec)
+        assert ctx.selected_relight_variant(prec, k, w * h) == kept
+        for _ in range(3):
+            best, ms = ctx.autotune_relight(scenes[1], env, frames[1], prec)
+            assert best == 5 and ms > 0
+            assert ctx.selected_relight_variant(prec, k, w * h) == kept
+    ctx.close()
