@@ -140,9 +140,8 @@ def test_cast_small_and_degenerate_meshes(nw, orc, ctx, nt):
 @pytest.mark.parametrize("leaf", [1, 3, 8])
 def test_cast_skewed_tree(nw, orc, ctx, leaf):
     # Groups of `leaf` parallel triangles whose size grows by 1.6 a group, all
-    # around one axis: the surface-area split peels one group off a level, so a
-    # ray near the axis leaves an entry on its stack at most levels of the
-    # tree and takes leaves of few triangles up to the largest.
+    # around one axis: an unbalanced tree (a third to a half of the depth bound)
+    # with leaves of few triangles up to the largest.
     base = np.array([[-1, -1, 0], [1, -1, 0], [0, 1.5, 0]], np.float64)
     v = np.concatenate([base * 0.05 * 1.6 ** i + [0, 0, -3 - 0.01 * 1.6 ** i - 0.002 * j]
                         for i in range(22) for j in range(leaf)])
@@ -156,6 +155,41 @@ def test_cast_skewed_tree(nw, orc, ctx, leaf):
     want = _oracle(orc, s, 41, 33)
     _compare(got, want)
     assert 4 <= info["bvh_depth"] <= 24
+
+
+def comb_scene(sign):
+    """25 groups of 8 triangles at z = sign 16.5^-i: with 16 bins the one far
+    group is alone in its bin at every level, so the tree peels a group a level
+    and its 24 internal levels reach the depth bound.  Every triangle has the
+    box [-1, 1]^2, so a ray from the other side of z = 0 meets both children of
+    every node, the rest first, and leaves the far group's leaf on its stack 24
+    times.  All but three triangles are slivers along the box's diagonal: what
+    is seen are the wide ones of the three farthest groups."""
+    v = []
+    for i in range(25):
+        z = sign * 16.5 ** -i
+        wide = {2: [[-1, -1], [1, 1], [1, -0.4]], 1: [[-1, -1], [1, 1], [-0.2, 1]],
+                0: [[-1, 1], [1, -1], [0.6, 0.7]]}.get(i)
+        for j in range(8):
+            t = wide if j == 0 and wide else [[-1, -1], [1, 1], [1e-5 * (j + 1), -1e-5]]
+            v += [[x, y, z] for x, y in t]
+    n = len(v) // 3
+    return {"vertices": np.array(v, np.float32),
+            "indices": np.arange(3 * n, dtype=np.int32).reshape(-1, 3),
+            "materials": np.array([[0.2, 0.3, 0.4, 0.0, 0.0, 0.0, 0.6, 0],
+                                   [0.7, 0.1, 0.4, 0.0, 0.0, 0.0, 0.6, 0]], np.float32),
+            "material_ids": (np.arange(n) // 8 % 2).astype(np.int32),
+            "camera": [0.0, 0.0, -2.5 * sign, 0.0, 0.0, 0.0, 0.0, 1.0, 0.0],
+            "bounds": np.array([-2, -2, -3, 2, 2, 3], np.float32)}
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_cast_tree_at_the_depth_bound(nw, orc, ctx, sign):
+    s = comb_scene(sign)
+    got, info = _cast(nw, ctx, s, 61, 47)
+    assert info["bvh_depth"] == 24
+    nh, nm = _compare(got, _oracle(orc, s, 61, 47), min_safe=0.95)  # the slivers' diagonal
+    assert nh > 800 and nm > 300
 
 
 def test_cast_null_fields_are_skipped(nw, ctx):
