@@ -106,6 +106,70 @@ def test_transfer_projection_tiles(nw, orc, ctx, deg, samples):
     ctx.mesh_destroy(mesh)
 
 
+@pytest.mark.parametrize("deg", [4, 5, 6])
+def test_transfer_nan_sample_scales_the_row(nw, ctx, deg):
+    """A sample whose radiance is NaN in one channel scales the column's rows
+    by 1 + 1 / samples in all three.  The NaN: maps whose blue is 1e38 and
+    -5e37 at every other texel, over panels that reflect 64 times the blue; where a
+    path meets both signs its blue is infinity minus infinity.  The same maps
+    with blue 2^-70 times as large take the same paths (the power of two leaves
+    the sampling tables as they are) and have no NaN, so calls of 1, 2, ...
+    samples on them give each sample's red and green term, and the rule applied
+    to the terms one after the other gives the rows of the first maps.  Up to 40
+    samples: past the projection's chunks of 32 and 16."""
+    N, nc = 40, (deg + 1) ** 2
+    v, ix, mids, mats, _ = panel_scene()
+    mats = [list(m) for m in mats]
+    mats[0][2] = mats[1][2] = 64.0
+    between = np.random.default_rng(1).uniform([-0.8, -0.8, 0.05], [0.8, 0.8, 0.55], (200, 3))
+    v = np.concatenate([v, between.astype(np.float32)])
+    maps = [0, 1, nc - 1]
+    mesh = _mesh(ctx, v, ix, mats, mids)
+    basis = smooth_basis(nc, seed=deg)
+    basis[..., 2] = np.where(np.arange(8) % 2 == 1, -5e37, 1e38)
+    small = basis.copy()
+    small[..., 2] *= np.float32(2.0 ** -70)
+
+    def calls(b):  # [sample count][v][k][map][red, green]
+        out = [np.zeros((len(v), nc, len(maps), 2))]
+        for n in range(1, N + 1):
+            T = _transfer(nw, ctx, mesh, b, deg, len(v), samples=n, seed=13)
+            out.append(T.reshape(len(v), nc, nc, 3)[:, :, maps, :2])
+        return np.array(out)
+
+    hot, ref = calls(basis), calls(small)
+    assert np.isfinite(hot).all() and np.isfinite(ref).all()
+    term = [(m + 1) * ref[m + 1] - m * ref[m] for m in range(N)]
+    # FP32 sums of up to 40 terms, and a term recovered from two of them.
+    size = np.abs(np.array(term)).sum(0).max() * 40 * 2.0 ** -23
+
+    def fold(count, nan, n):
+        acc = np.zeros_like(ref[0])
+        for m in range(count):
+            acc = np.where(nan[m][:, None, :, None], acc * (1 + 1 / n), acc + term[m] / n)
+        return acc
+
+    nan = []  # [sample][v][i], found from the call in which the sample is the last
+    for m in range(N):
+        before = fold(m, nan, m + 1)
+        got = hot[m + 1]
+        as_nan = np.abs(got - before * (1 + 1 / (m + 1))).max(axis=(1, 3))
+        as_term = np.abs(got - (before + term[m] / (m + 1))).max(axis=(1, 3))
+        nan.append(as_nan < as_term)
+        assert np.minimum(as_nan, as_term).max() <= size, (m, np.minimum(as_nan, as_term).max())
+    nan = np.array(nan)
+    print(f"deg {deg}: {nan.mean():.4f} of samples NaN, at the chunks' ends "
+          f"{[int(nan[m].sum()) for m in (15, 16, 31, 32)]}")
+    assert all(nan[m].any() for m in (15, 16, 31, 32))
+    changed = 0
+    for n in (16, 17, 32, 33, N):
+        want = fold(n, nan, n)
+        assert np.abs(hot[n] - want).max() <= size, (n, np.abs(hot[n] - want).max())
+        changed += (np.abs(want - ref[n]) > 100 * size).sum()
+    assert changed > 1000  # the rule mattered
+    ctx.mesh_destroy(mesh)
+
+
 def test_transfer_with_vertex_normals_replays_oracle(nw, orc, ctx):
     """Smooth-shaded geometry: a faceted bowl (interpolated normals differ
     from the geometric ones) with a floor; degree 2, 384 samples."""
