@@ -53,15 +53,15 @@ typedef enum {
 
 /* Arithmetic of the per-(pixel, wavelet) MLP. */
 typedef enum {
-  NWPRT_PREC_FP32 = 0, /* plain form: FP32 vector ALU, one pixel per lane    */
+  NWPRT_PREC_FP32 = 0, /* plain form: FP32 operands, products and sums, on the
+                          FP32 matrix instructions                           */
   NWPRT_PREC_FP16 = 1, /* fused MFMA, FP16 operands, FP32 accumulation       */
   NWPRT_PREC_BF16 = 2, /* fused MFMA, BF16 operands, FP32 accumulation       */
   NWPRT_PREC_FP8 = 3   /* fused MFMA: hidden layers FP8-E4M3 (OCP) with one
                           power-of-two scale per layer, weights from their
                           amax, activations from a BF16 calibration launch
-                          over ~8K pixels of the frame; first layer BF16;
-                          FP32 accumulation.  Scenes with aux inputs:
-                          NWPRT_ERR_UNSUPPORTED. */
+                          over ~16K pixels of the frame; first layer BF16;
+                          FP32 accumulation. */
 } nwprt_precision;
 
 typedef enum { NWPRT_DTYPE_F32 = 0, NWPRT_DTYPE_F16 = 1 } nwprt_dtype;
@@ -735,8 +735,8 @@ nwprt_status nwprt_debug_transport(nwprt_ctx ctx, int32_t scene_id,
  * tile variant.  The graph reads the G-buffers, environment-map selections
  * and outputs through the pointers given here, so new contents (e.g. an
  * nwprt_envmap_update_faces of a job's map, same K) are picked up by the
- * next launch.  BF16 / FP16 only; scenes without aux inputs; all jobs must
- * share the output activation (NWPRT_ERR_UNSUPPORTED otherwise). */
+ * next launch.  BF16, FP16 or FP8; all jobs must share the output activation
+ * (NWPRT_ERR_UNSUPPORTED otherwise). */
 typedef struct {
   int32_t scene_id;
   int32_t env_id;

@@ -20,10 +20,12 @@
 //
 // What bounds it: the FP32 matrix rate (64 FLOP per cycle and SIMD, 157 TFLOP/s
 // nominal; a large FP32 matrix product measures 152).  The weights stay in
-// LDS (44 KB, shared by four waves; 40 16-byte reads per wavelet against 5 K
-// matrix cycles per 16 pixels), so registers hold only activations.  960 x 540,
-// K = 64 (33 M pairs, 692 GFLOP): 5.25 ms, 132 TFLOP/s; with one lane per
-// pixel on the vector ALU and one LDS read per four products it was 21.1 ms.
+// LDS (40 KB, shared by four waves; 40 16-byte reads per wavelet against 5 K
+// matrix cycles per 16 pixels; the output layer's stay in 16 registers), so
+// the other registers hold activations.  960 x 540, K = 64 (33 M pairs, 692
+// GFLOP): 5.30 ms, 131 TFLOP/s, the matrix cores busy for 85 % of the cycles;
+// with one lane per pixel on the vector ALU and one LDS read per four products
+// it was 21.0 ms.
 #include <hip/hip_runtime.h>
 
 #include "device_common.hpp"
